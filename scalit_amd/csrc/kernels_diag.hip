@@ -9,6 +9,9 @@
 //   |d offdiag| <= tol * initial or BJMAX sweeps (hosbdiag.f90:5-75);
 //   VOSB accumulates the rotations (vupdate.f90:21-36), EIG0 <- diag(HOSB).
 //
+// Real separable levels of up to 128 points: kernels_jacobi.hip.  The others
+// (complex level matrices, the dense sNDVR layer, larger levels) here:
+//
 // Level 1 (NDK = 1): one wave per block runs the whole Jacobi in LDS.
 // Levels with NDK > 1: one launch per rotation; each workgroup owns a slice of
 // 64 inner points d (its 4 waves split the rotated rows and columns), reduces
@@ -627,7 +630,10 @@ int block_diag(scalit_ctx *c, int bjmax, double bjtol)
     HIP_TRY(hipMemcpyAsync(c->eig0.p, c->res.p, sizeof(double) * c->N, hipMemcpyDeviceToDevice, s));
     for (int l = c->sF - 1; !c->scx && l >= 0; l--) {
         Level &L = c->lv[l];
-        if (L.dim == 1 && sizeof(double) * (size_t)L.n * L.n > 160 * 1024) {
+        const bool layer = c->ndvr && l == c->sF - 1;
+        if (L.dim == 1 && !layer && jacobi_vec_fits(L.n)) {
+            SC_TRY(jacobi_level_vec(c, l, bjmax, bjtol, s));
+        } else if (L.dim == 1 && sizeof(double) * (size_t)L.n * L.n > 160 * 1024) {
             SC_TRY(diag_level_dense(c, l, s));
         } else if (L.dim == 1) {
             size_t lds = sizeof(double) * (size_t)L.n * L.n;
@@ -636,9 +642,11 @@ int block_diag(scalit_ctx *c, int bjmax, double bjtol)
                                c->eig0.p, L.vosb.p, bjmax, bjtol, (int *)nullptr);
             HIP_TRY(hipGetLastError());
             HIP_TRY(hipStreamSynchronize(s));
+        } else if (!layer && jacobi_block_fits(L.n)) {
+            SC_TRY(jacobi_level_block(c, l, bjmax, bjtol, s));
         } else {
-            SC_TRY(diag_level_ndk<double>(c, l, bjmax, bjtol, (c->ndvr && l == c->sF - 1) ? c->outh.p : nullptr,
-                                          L.h0.p, L.dep ? L.depv.p : nullptr, s));
+            SC_TRY(diag_level_ndk<double>(c, l, bjmax, bjtol, layer ? c->outh.p : nullptr, L.h0.p,
+                                          L.dep ? L.depv.p : nullptr, s));
         }
     }
     if (c->scx) SC_TRY(block_diag_cx(c, bjmax, bjtol, s));

@@ -240,6 +240,12 @@ void osbw_scatter(scalit_ctx *c, int nvec, double *y, long ldy, const int *activ
 
 // OSB set-up (kernels_diag.hip)
 int block_diag(scalit_ctx *c, int bjmax, double bjtol);
+// one level of it for a real separable level (kernels_jacobi.hip): NDK = 1, or
+// NDK > 1; VOSB of the level is written, EIG0 updated, the stream waited for
+bool jacobi_vec_fits(int n);
+int jacobi_level_vec(scalit_ctx *c, int l, int bjmax, double bjtol, hipStream_t s);
+bool jacobi_block_fits(int n);
+int jacobi_level_block(scalit_ctx *c, int l, int bjmax, double bjtol, hipStream_t s);
 // symmetric eigen-solve of a small dense matrix on the GPU (one workgroup).
 // a: n x n device, lda; w: n device (ascending); z: eigenvectors (device, ldz) or nullptr
 int small_sym_eig(int n, const double *a, int lda, double *w, double *z, int ldz, double *work, hipStream_t s);

@@ -1,0 +1,83 @@
+"""The OSB set-up's joint Jacobi on the GPU against the oracle's restatement
+of HosbDiag / MJACOBI at the sizes where its kernels change: tile edges and
+remainders, one-point levels, the R factor of the joint matrices (one chunk,
+several rounds, chunks in LDS and in memory), U in LDS or in memory, levels
+past the new kernels' sizes, levels with and without DEP, two to four levels.
+
+Tolerances (those of the other set-up tests): EIG0 1e-9, VOSB 1e-7, both
+relative to the largest entry.  The oracle's own sensitivity to a 1e-15
+relative change of RES is 1e-11 in VOSB; with a stopping tolerance of 1e-5
+the two run the same sweeps unless the measure's change lies within rounding
+of it.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from scalit_amd import problems as P
+from scalit_amd.context import Context
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(sN, h0, dep, res, bjmax=1000, bjtol=1e-5):
+    op = O.Operator(sN, h0, res, dep)
+    vo, eo = op.diag(bjmax, bjtol)
+    ctx = Context(sN, [d is not None for d in dep])
+    for l, h in enumerate(h0):
+        ctx.set_h0(l + 1, h)
+        if dep[l] is not None:
+            ctx.set_dep(l + 1, dep[l])
+    ctx.set_res(res)
+    ctx.block_diag(bjmax, bjtol)
+    v, e = ctx.get_precond()
+    errs = [float(np.abs(a - b).max()) for a, b in zip(v, vo)]
+    ee = float(np.abs(e - eo).max() / np.abs(eo).max())
+    print(sN, "VOSB", errs, "EIG0", ee, flush=True)
+    assert ee <= 1e-9
+    assert max(errs) <= 1e-7
+    for l, n in enumerate(sN):   # the last block's rotation stays orthogonal
+        w = v[l][-n * n:].reshape(n, n, order="F")
+        assert np.abs(w.T @ w - np.eye(n)).max() <= 1e-12
+    ctx.close()
+
+
+@pytest.mark.parametrize("grid", [
+    (5, 3, 2),        # one tile of everything
+    (2, 1, 1),        # one-point levels
+    (16, 17, 3),      # a tile and one more
+    (33, 31, 7),      # odd sizes below and above a tile
+    (48, 16, 40),     # level 3: R factor in two rounds, chunks in LDS
+    (40, 65, 4),      # five tiles along level 2, fewer points than its size
+    (3, 100, 9),      # U in memory
+    (20, 9, 97),      # R factor (180 > 98) with U in memory
+    (30, 20, 110),    # R factor in two rounds, chunks in memory
+    (101, 3, 2),      # level 1 with V in memory
+    (128, 2, 2),      # its largest size
+    (140, 2, 2),      # level 1 past it: one wave per block
+    (8, 6, 129),      # level 3 past it: one launch per rotation
+])
+def test_setup_matches_oracle(grid):
+    prob = P.build_problem(*grid, P.gaussian_potential(17), seed=17)
+    _check(prob.sN, prob.h0, prob.dep, prob.res)
+
+
+@pytest.mark.parametrize("sN,deps", [((7,), ()), ((12, 9), (1,)), ((12, 9), ()), ((6, 5, 4, 7), (1, 3)),
+                                     ((10, 4, 11), ())])
+def test_setup_other_levels(sN, deps):
+    """Seeded symmetric level matrices, DEP on the levels of `deps`."""
+    g = P.rng(5)
+    h0, dep, dim = [], [], 1
+    for l, n in enumerate(sN):
+        a = g.standard_normal((n, n))
+        h0.append(0.05 * (a + a.T) + np.diag(np.arange(n, dtype=float)))
+        dep.append(g.uniform(0.5, 1.5, size=dim) if l in deps else None)
+        dim *= n
+    _check(sN, h0, dep, g.standard_normal(dim))
+
+
+@pytest.mark.parametrize("bjmax,bjtol", [(0, 1e-5), (1, 1e-5), (3, 0.0), (1000, 1e-9)])
+def test_setup_stopping(bjmax, bjtol):
+    """No sweep, one, a fixed count (tolerance 0), and a tight tolerance."""
+    prob = P.build_problem(18, 20, 9, P.gaussian_potential(23), seed=23)
+    _check(prob.sN, prob.h0, prob.dep, prob.res, bjmax, bjtol)
