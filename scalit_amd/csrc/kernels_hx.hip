@@ -4,8 +4,9 @@
 // (H1X / H2X) and the block loops of src/iterate/libiterate/hpx/hpx.f90:5-35.
 //
 // Two paths:
-//  * generic: any number of levels and DEP pattern; one accumulate-kernel per
-//    level (thread per output element).
+//  * generic: any number of levels and DEP pattern; the diagonal and levels 1
+//    and 2 in one MFMA pass, then one accumulate-kernel per further level
+//    (thread per output element).
 //  * fused 3-level path for sF=3, sDEP=(F,F,T) -- r, R, theta with
 //    DEP(r,R) x L^2_theta -- on FP64 / FP32 MFMA:
 //      pass A, one workgroup per (theta point, vector) slab S(n1 x n2) staged
@@ -21,6 +22,7 @@
 #include <cstdlib>
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "device_common.hpp"
 #include "outer_mode.hpp"
@@ -49,12 +51,11 @@ __global__ void k_diag_init(long n, const T *__restrict__ res, const T *__restri
         st_cvt<T, S>(yv, i, (res[i] - s) * ld_cvt<T, S>(xv, i));
 }
 
-// Y(k, i, b) += sum_j H(i,j) [DEP(k)] X(k, j, b)     (H1X_XYZ / H1X_DEP)
-// transpose: H(j,i) instead (the adjoint).
+// Y(k, i, b) += sum_j H(i,j) [DEP(k)] X(k, j, b)     (H1X_XYZ / H1X_DEP; the
+// adjoint passes the transposed copy of H)
 template <typename T, typename S>
 __global__ void k_mode_generic(int nin, int nout, int blk, const T *__restrict__ h, const T *__restrict__ dep,
-                               bool transpose, const S *__restrict__ x, long ldx, S *__restrict__ y, long ldy,
-                               const int *active)
+                               const S *__restrict__ x, long ldx, S *__restrict__ y, long ldy, const int *active)
 {
     int v = blockIdx.y;
     if (!vec_active(active, v)) return;
@@ -68,11 +69,7 @@ __global__ void k_mode_generic(int nin, int nout, int blk, const T *__restrict__
         long b = t / nout;
         const S *xb = xv + b * (long)nin * nout + k;
         T acc = 0;
-        if (transpose) {
-            for (int j = 0; j < nout; j++) acc += h[j + (long)nout * i] * ld_cvt<T, S>(xb, (long)nin * j);
-        } else {
-            for (int j = 0; j < nout; j++) acc += h[i + (long)nout * j] * ld_cvt<T, S>(xb, (long)nin * j);
-        }
+        for (int j = 0; j < nout; j++) acc += h[i + (long)nout * j] * ld_cvt<T, S>(xb, (long)nin * j);
         if (dep) acc *= dep[k];
         st_cvt<T, S>(yv, idx, ld_cvt<T, S>(yv, idx) + acc);
     }
@@ -169,29 +166,226 @@ static const T *outh_of(const scalit_ctx *c)
     else return (const T *)c->outh_f.p;
 }
 
+// ---------------------------------------------------------------------------
+// levels 1 and 2 of the generic path in one pass
+//   Y(i,c) = (RES(i,c) - s) X(i,c) + sum_j H1(i,j) X(j,c) + DEP(i) sum_j H2(c,j) X(i,j)
+// for every (n1 x n2) plane of every vector, on MFMA.  One wave per 16 x 16
+// output tile and, when there are few tiles, KSPL waves of a workgroup per
+// tile, each a share of both sums (added through LDS): the truncated operator
+// (n1 = 400, n2 = 96) has only 150 tiles per vector, so what counts is one
+// tile's chain of MFMAs, not operand reuse.  Tiles are computed transposed (D =
+// Y^T, as in the 3-level path) so that every access of H1, H2, RES, Y and the
+// second sum's X runs along lanes; the first sum's X, whose contiguous index
+// is the summed one, goes through LDS in chunks of LV_KC rows (read straight
+// into fragments it costs one cache line per lane: 15 us instead of 12 at
+// n1 = 400, n2 = 96, 4 vectors; 95 us as the diagonal and one accumulate pass of a
+// thread per value for each level).  Two chunks and four groups of each sum's
+// operands are in flight, by buffer loads (one 32-bit addition of address each), every load issued on every
+// path so that the waits count exactly; loads past the end return zero.
+constexpr int LV_KC = 64;
+
+template <typename T, typename S, int KSPL>
+__global__ void __launch_bounds__(256) k_hx_levels12(int n1, int n2, int nvec, const T *__restrict__ h1,
+                                                     const T *__restrict__ h2, const T *__restrict__ dep2,
+                                                     const T *__restrict__ res, const T *__restrict__ shifts, T shift0,
+                                                     const S *__restrict__ x, long ldx, S *__restrict__ y, long ldy,
+                                                     const int *__restrict__ active)
+{
+    using M = Mfma<T>;
+    using acc_t = typename M::acc_t;
+    constexpr int TI = KSPL == 4 ? 1 : 2, TC = KSPL == 1 ? 2 : 1;   // tiles of a workgroup along i and c
+    constexpr int GC = LV_KC / 16 / KSPL;                           // groups of 16 k per wave and chunk
+    constexpr int PF = 4, PF2 = 2;                                  // groups in flight of each sum
+    constexpr int LDX = LV_KC + 1, NST = 16 * TC * LV_KC / 256;
+    constexpr int ST = (int)sizeof(T), SS = (int)sizeof(S);
+    __shared__ T sx[2][16 * TC * LDX];   // X(k0 + k, c) at k + LDX c
+    const int v = (int)(blockIdx.z % (unsigned)nvec);
+    const long b = blockIdx.z / (unsigned)nvec;
+    if (!vec_active(active, v)) return;   // the same for the whole workgroup
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 15, lk = lane >> 4;
+    const int tile = wave / KSPL, ks = wave % KSPL;
+    const int ti = (int)blockIdx.x * TI + tile % TI, tcl = tile / TI, tc = (int)blockIdx.y * TC + tcl;
+    const int P = n1 * n2;
+    const S *xp = x + (long)v * ldx + (long)P * b;
+    const int i = min(ti * 16 + lr, n1 - 1), ca = min(tc * 16 + lr, n2 - 1);   // B column, A row of this lane
+    // loads past the end of a matrix or of the plane return zero
+    const auto rx = buf_rsrc(xp, (long)P * SS), rh1 = buf_rsrc(h1, (long)n1 * n1 * ST),
+               rh2 = buf_rsrc(h2, (long)n2 * n2 * ST), rr = buf_rsrc(res + (long)P * b, (long)P * ST);
+
+    // first sum, A(c,k) = X(k,c) from LDS, B(k,i) = H1(i,k): group g covers
+    // k = 16 g..16 g + 15, wave share ks the groups ks, ks + KSPL, ...
+    const int xk = tid & (LV_KC - 1), xc = tid / LV_KC;
+    const int xv = (xk + n1 * ((int)blockIdx.y * 16 * TC + xc)) * SS, xstep = n1 * (256 / LV_KC) * SS;
+    auto load_x = [&](int k0, T(&r)[NST]) {
+#pragma unroll
+        for (int u = 0; u < NST; u++) r[u] = buf_ld<T, S>(rx, xv + k0 * SS + u * xstep, 0);
+    };
+    auto stage_x = [&](int k0, const T(&r)[NST], T *d) {   // a k past the end has read the next column
+#pragma unroll
+        for (int u = 0; u < NST; u++) d[xk + LDX * (xc + 256 / LV_KC * u)] = k0 + xk < n1 ? r[u] : (T)0;
+    };
+    const int hv = (i + n1 * lk) * ST;
+    auto load_h = [&](int g, T(&r)[4]) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) r[u] = buf_ld<T, T>(rh1, hv + n1 * (16 * g + 4 * u) * ST, 0);
+    };
+    // second sum, A(c,j) = H2(c,j), B(j,i) = X(i,j)
+    const int gv = (ca + n2 * lk) * ST, yv = (i + n1 * lk) * SS;
+    const int G2 = (n2 + 15) / 16;
+    auto load2 = [&](int g, T(&ra)[4], T(&rb)[4]) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            ra[u] = buf_ld<T, T>(rh2, gv + n2 * (16 * g + 4 * u) * ST, 0);
+            rb[u] = buf_ld<T, S>(rx, yv + n1 * (16 * g + 4 * u) * SS, 0);
+        }
+    };
+    T st[2][NST], hb[PF][4], qa[PF2][4], qb[PF2][4];
+    load_x(0, st[0]);
+    load_x(LV_KC, st[1]);
+#pragma unroll
+    for (int u = 0; u < PF; u++) load_h(ks + KSPL * u, hb[u]);
+    // the diagonal's term
+    T rv[4], xd[4];
+    const int ov = (i + n1 * (tc * 16 + M::row(lk, 0)));
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        rv[q] = buf_ld<T, T>(rr, (ov + n1 * M::row(0, q)) * ST, 0);
+        xd[q] = buf_ld<T, S>(rx, (ov + n1 * M::row(0, q)) * SS, 0);
+    }
+    const T sh = shifts ? shifts[v] : shift0, d2 = dep2 ? dep2[i] : (T)1;
+#pragma unroll
+    for (int u = 0; u < PF2; u++) load2(ks + KSPL * u, qa[u], qb[u]);
+    acc_t acc = acc_t{0, 0, 0, 0}, acc2 = acc_t{0, 0, 0, 0};
+    const int nch = (n1 + LV_KC - 1) / LV_KC;
+    stage_x(0, st[0], sx[0]);
+    // chunk ch from its LDS buffer, while chunk ch + 2 loads into the registers that staged it
+    // and chunk ch + 1 goes to the other buffer
+    auto chunk = [&](int ch, T(&mine)[NST], const T(&next)[NST], const T *cur, T *other, auto hslot) {
+        __syncthreads();   // chunk ch is staged, and the other buffer read by all
+        load_x(LV_KC * (ch + 2), mine);
+        const T *sc = cur + LDX * (16 * tcl + lr) + 16 * ks + lk;
+        const int g0 = ch * (LV_KC / 16) + ks;
+#pragma unroll
+        for (int u = 0; u < GC; u++) {
+            constexpr int H0 = decltype(hslot)::value;
+#pragma unroll
+            for (int w = 0; w < 4; w++)
+                acc = M::run(sc[16 * KSPL * u + 4 * w], hb[(H0 + u) % PF][w], acc);
+            load_h(g0 + KSPL * (u + PF), hb[(H0 + u) % PF]);
+        }
+        stage_x(LV_KC * (ch + 1), next, other);
+    };
+    // four chunks at a time: the slot of a group's H1 values is a constant
+    int ch = 0;
+    for (; ch + 4 <= nch; ch += 4) {
+        chunk(ch, st[0], st[1], sx[0], sx[1], std::integral_constant<int, 0>());
+        chunk(ch + 1, st[1], st[0], sx[1], sx[0], std::integral_constant<int, GC % PF>());
+        chunk(ch + 2, st[0], st[1], sx[0], sx[1], std::integral_constant<int, 2 * GC % PF>());
+        chunk(ch + 3, st[1], st[0], sx[1], sx[0], std::integral_constant<int, 3 * GC % PF>());
+    }
+    if (ch < nch) chunk(ch, st[0], st[1], sx[0], sx[1], std::integral_constant<int, 0>());
+    if (ch + 1 < nch) chunk(ch + 1, st[1], st[0], sx[1], sx[0], std::integral_constant<int, GC % PF>());
+    if (ch + 2 < nch) chunk(ch + 2, st[0], st[1], sx[0], sx[1], std::integral_constant<int, 2 * GC % PF>());
+    {
+        const int G = (G2 - ks + KSPL - 1) / KSPL;   // groups of this share
+        int g = 0;
+        for (; g + PF2 <= G; g += PF2) {
+#pragma unroll
+            for (int u = 0; u < PF2; u++) {
+#pragma unroll
+                for (int w = 0; w < 4; w++) acc2 = M::run(qa[u][w], qb[u][w], acc2);
+                load2(ks + KSPL * (g + u + PF2), qa[u], qb[u]);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < PF2 - 1; u++)
+            if (g + u < G)
+#pragma unroll
+                for (int w = 0; w < 4; w++) acc2 = M::run(qa[u][w], qb[u][w], acc2);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) acc[q] += d2 * acc2[q];
+    if constexpr (KSPL > 1) {
+        T *red = sx[0];
+        __syncthreads();   // the last chunk is read
+#pragma unroll
+        for (int q = 0; q < 4; q++) red[256 * wave + 64 * q + lane] = acc[q];
+        __syncthreads();
+        if (ks != 0) return;   // no barrier follows
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            for (int k = 1; k < KSPL; k++) acc[q] += red[256 * (wave + k) + 64 * q + lane];
+    }
+    const auto ry = buf_rsrc(y + (long)v * ldy + (long)P * b, (long)P * SS);
+    // rows past the last c lie past the plane and are dropped
+    if (ti * 16 + lr < n1)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            buf_st<T, S>(ry, (ov + n1 * M::row(0, q)) * SS, 0, acc[q] + (rv[q] - sh) * xd[q]);
+}
+
+// KSPL: 1, 2 or 4 waves per tile, as many as leave about one wave per SIMD.
+// FP64, us with 1 / 2 / 4 waves: n1 = 400, n2 = 96 (150 tiles a vector): 1 vector 11.7 /
+// 8.0 / 7.4, 2 vectors 11.8 / 8.0 / 9.4, 4 vectors 12.0 / 12.2 / 12.2; n1 = 1000,
+// n2 = 64 (252 tiles): 1 vector 20 / 13 / 10, 8 vectors 34 / 39 / 53.
+template <typename T, typename S>
+static void launch_levels12(int n1, int n2, int nplane, int nvec, const T *h1, const T *h2, const T *dep2,
+                            const T *res, const T *shifts, T shift0, const S *x, long ldx, S *y, long ldy,
+                            const int *active, hipStream_t s)
+{
+    const int nti = (n1 + 15) / 16, ntc = (n2 + 15) / 16;
+    const long simds = 4L * g_num_cu, tiles = (long)nti * ntc * nplane * nvec;
+#define LV(K, TI, TC)                                                                                           \
+    hipLaunchKernelGGL((k_hx_levels12<T, S, K>), dim3((nti + TI - 1) / TI, (ntc + TC - 1) / TC, nplane *nvec), \
+                       dim3(256), 0, s, n1, n2, nvec, h1, h2, dep2, res, shifts, shift0, x, ldx, y, ldy, active)
+    if (4 * tiles <= simds) LV(4, 1, 1);
+    else if (2 * tiles <= simds) LV(2, 2, 1);
+    else LV(1, 2, 2);
+#undef LV
+}
+
+// 32-bit byte offsets within a plane and a level matrix (the loads in flight
+// reach less than 1,024 indices past them), the grid's z range
+static bool levels12_fits(long n1, long n2, long nplane, long nvec, size_t item)
+{
+    return (std::max(n1, n2) + 1024) * (std::max(n1, n2) + 1024) * (long)item < 0x7fffffffL && nplane * nvec <= 65535;
+}
+
 template <typename T, typename S>
 static int hx_generic(scalit_ctx *c, const T *res, const T *shifts, T shift0, int nvec, const S *x, long ldx, S *y,
                       long ldy, bool transpose, const int *active, hipStream_t s)
 {
     const int th = 256;
     dim3 g(grid_for(c->N, th), nvec);
-    hipLaunchKernelGGL((k_diag_init<T, S>), g, dim3(th), 0, s, c->N, res, shifts, shift0, x, ldx, y, ldy, active);
+    const T *h[SC_FMAX], *dep[SC_FMAX];
     for (int l = 0; l < c->sF; l++) {
         const Level &L = c->lv[l];
-        if (c->ndvr && l == c->sF - 1) {
-            launch_h3x<T, S>(L.dim, L.n, nvec, outh_of<T>(c), transpose, x, ldx, y, ldy, active, s);
-            continue;
-        }
-        const T *h, *dep = nullptr;
         if constexpr (sizeof(T) == 8) {
-            h = (const T *)(transpose ? L.h0t.p : L.h0.p);
-            if (L.dep) dep = (const T *)L.depv.p;
+            h[l] = (const T *)(transpose ? L.h0t.p : L.h0.p);
+            dep[l] = L.dep ? (const T *)L.depv.p : nullptr;
         } else {
-            h = (const T *)L.h0_f.p;   // the fp32 copies serve the forward product only
-            if (L.dep) dep = (const T *)L.depv_f.p;
+            h[l] = (const T *)L.h0_f.p;   // the fp32 copies serve the forward product only
+            dep[l] = L.dep ? (const T *)L.depv_f.p : nullptr;
         }
-        hipLaunchKernelGGL((k_mode_generic<T, S>), g, dim3(th), 0, s, L.dim, L.n, L.blk, h, dep, transpose, x, ldx,
-                           y, ldy, active);
+    }
+    // the diagonal and levels 1 and 2 in one pass where both are level matrices
+    int l = 0;
+    const Level *L = c->lv;
+    if (c->sF >= 2 + (c->ndvr ? 1 : 0) && levels12_fits(L[0].n, L[1].n, L[1].blk, nvec, sizeof(T))) {
+        launch_levels12<T, S>(L[0].n, L[1].n, L[1].blk, nvec, h[0], h[1], dep[1], res, shifts, shift0, x, ldx, y,
+                              ldy, active, s);
+        l = 2;
+    } else {
+        hipLaunchKernelGGL((k_diag_init<T, S>), g, dim3(th), 0, s, c->N, res, shifts, shift0, x, ldx, y, ldy, active);
+    }
+    for (; l < c->sF; l++) {
+        if (c->ndvr && l == c->sF - 1)
+            launch_h3x<T, S>(L[l].dim, L[l].n, nvec, outh_of<T>(c), transpose, x, ldx, y, ldy, active, s);
+        else
+            hipLaunchKernelGGL((k_mode_generic<T, S>), g, dim3(th), 0, s, L[l].dim, L[l].n, L[l].blk, h[l], dep[l],
+                               x, ldx, y, ldy, active);
     }
     HIP_TRY(hipGetLastError());
     return SCALIT_OK;

@@ -1,0 +1,111 @@
+"""H*X of the generic path (any number of levels and DEP pattern) at the edges
+of its first pass, levels 1 and 2 with the diagonal on MFMA tiles: one-point
+levels, tile edges and remainders, k remainders, one, two and four waves per
+tile, several planes, with and without DEP, nonsymmetric level matrices
+forward and adjoint, FP64 / FP32 / BF16 storage, and per-vector shifts.
+
+Reference: dense mode products in FP64 (numpy) of the values the device
+holds.  Tolerances relative to the largest entry: FP64 1e-12 (the parity bound
+of the other H*X tests), FP32 2e-6 and BF16 storage 2e-2 likewise.
+"""
+import numpy as np
+import pytest
+import torch
+
+from scalit_amd import _lib as L
+from scalit_amd import problems as P
+from scalit_amd.context import Context
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    ((1, 1), (), 1),
+    ((2, 3), (1,), 2),
+    ((16, 16), (), 1),
+    ((17, 33), (1,), 3),
+    ((400, 96), (1,), 1),      # four waves per tile
+    ((400, 96), (1,), 2),      # two
+    ((400, 96), (1,), 5),      # one
+    ((5, 130), (), 7),
+    ((259, 2), (), 4),
+    ((31, 5, 4), (), 2),
+    ((20, 18, 7), (1, 2), 9),
+    ((6, 5, 4, 7), (1, 3), 3),
+]
+
+
+def _operator(sN, deps, seed=3):
+    g = P.rng(seed)
+    h0, dep, dim = [], [], 1
+    for l, n in enumerate(sN):
+        h0.append(g.standard_normal((n, n)) / np.sqrt(n))
+        dep.append(g.uniform(0.5, 1.5, size=dim) if l in deps else None)
+        dim *= n
+    res = g.standard_normal(dim)
+    ctx = Context(sN, [d is not None for d in dep])
+    for l, h in enumerate(h0):
+        ctx.set_h0(l + 1, h)
+        if dep[l] is not None:
+            ctx.set_dep(l + 1, dep[l])
+    ctx.set_res(res)
+    return ctx, h0, dep, res
+
+
+def _reference(h0, dep, res, x, shifts, trans=False):
+    y = (res[None, :] - np.asarray(shifts).reshape(-1, 1)) * x
+    inner = 1
+    for h, d in zip(h0, dep):
+        n = h.shape[0]
+        z = np.einsum("ij,ajk->aik", h.T if trans else h, x.reshape(-1, n, inner))
+        if d is not None:
+            z = z * d
+        y = y + z.reshape(x.shape)
+        inner *= n
+    return y
+
+
+def _rel(a, b):
+    return float(np.abs(a - b).max() / np.abs(b).max())
+
+
+@pytest.mark.parametrize("sN,deps,nvec", SHAPES)
+def test_generic_levels(sN, deps, nvec):
+    L.lib().scalit_debug_force_generic(1)
+    try:
+        ctx, h0, dep, res = _operator(sN, deps)
+        ctx.set_shift(0.37)
+        x = P.random_vectors(ctx.N, nvec, 9)
+        xd = ctx.to_device(x)
+        assert _rel(ctx.hx(xd).cpu().numpy(), _reference(h0, dep, res, x, 0.0)) <= 1e-12
+        sh = np.linspace(-0.5, 0.5, nvec)
+        assert _rel(ctx.hx(xd, shifts=sh).cpu().numpy(), _reference(h0, dep, res, x, sh)) <= 1e-12
+        dx, dv = ctx.hx_adjoint(xd, ctx.to_device(x[::-1].copy()), L.TA1)
+        assert _rel(dx.cpu().numpy(), _reference(h0, dep, res, x[::-1], 0.37, True)) <= 1e-12
+        for dt, tol in ((torch.float32, 2e-6), (torch.bfloat16, 2e-2)):
+            xl = ctx.to_device(x, dt)
+            y = ctx.hx_lp(xl, L.TA1).double().cpu().numpy()
+            assert _rel(y, _reference(h0, dep, res, xl.double().cpu().numpy(), 0.37)) <= tol, dt
+        ctx.close()
+    finally:
+        L.lib().scalit_debug_force_generic(0)
+
+
+def test_generic_strided_vectors():
+    """Leading dimensions larger than N and a base that is only 8-byte aligned."""
+    ctx, h0, dep, res = _operator((37, 21), (1,))
+    n, ld = ctx.N, ctx.N + 5
+    x = P.random_vectors(n, 3, 11)
+    buf = torch.full((3 * ld + 1,), 7.0, dtype=torch.float64, device=ctx.dev)
+    out = torch.full((3 * ld + 1,), 5.0, dtype=torch.float64, device=ctx.dev)
+    for v in range(3):
+        buf[1 + v * ld:1 + v * ld + n] = ctx.to_device(x[v])[0]
+    import ctypes as C
+    L.check(L.lib().scalit_hx(ctx.handle, L.TA0, 3, C.c_void_p(buf.data_ptr() + 8), ld, C.c_void_p(out.data_ptr() + 8),
+                              ld, None, C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    o = out.cpu().numpy()
+    ref = _reference(h0, dep, res, x, 0.0)
+    for v in range(3):
+        assert _rel(o[1 + v * ld:1 + v * ld + n], ref[v]) <= 1e-12
+        assert (o[1 + v * ld + n:1 + (v + 1) * ld] == 5.0).all()
+    assert o[0] == 5.0
+    ctx.close()
