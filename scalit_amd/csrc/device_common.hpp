@@ -74,9 +74,10 @@ __device__ __forceinline__ T px_kernel(int nosb, T y, T eig, T e0, T de, T beta)
 __device__ __forceinline__ bool vec_active(const int *active, int v) { return active == nullptr || active[v] != 0; }
 
 // Targets of an address select that makes an optional load unconditional:
-// an activity flag for "every vector active" and the unit factor.
+// an activity flag for "every vector active", the unit factor and zero.
 static __device__ const int k_all_on = 1;
 static __device__ const double k_unit_d = 1.0;
+static __device__ const double k_zero_d = 0.0;
 static __device__ const float k_unit_f = 1.0f;
 template <typename T>
 __device__ __forceinline__ const T *unit_ptr()
