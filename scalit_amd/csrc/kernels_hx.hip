@@ -19,6 +19,8 @@
 //    of RB x CB output tiles at once (independent MFMA chains, fragment
 //    reuse); the block shape and wave count of each pass are chosen per
 //    problem and batch size by timing the candidates on the device (autotune).
+//    Small batches and grids take levels 1 and 2 tile by tile, and small ones
+//    the whole operator in one launch.
 #include <cstdlib>
 #include <algorithm>
 #include <cstring>
@@ -182,9 +184,13 @@ static const T *outh_of(const scalit_ctx *c)
 // thread per value for each level).  Two chunks and four groups of each sum's
 // operands are in flight, by buffer loads (one 32-bit addition of address each), every load issued on every
 // path so that the waits count exactly; loads past the end return zero.
+//
+// ONE (the 3-level operator, level 2 without DEP): one chain of products for
+// both sums and one wave per tile, the slab pass's order of additions, so that the
+// variants the autotuner picks from agree to the last bit.
 constexpr int LV_KC = 64;
 
-template <typename T, typename S, int KSPL>
+template <typename T, typename S, int KSPL, bool ONE>
 __global__ void __launch_bounds__(256) k_hx_levels12(int n1, int n2, int nvec, const T *__restrict__ h1,
                                                      const T *__restrict__ h2, const T *__restrict__ dep2,
                                                      const T *__restrict__ res, const T *__restrict__ shifts, T shift0,
@@ -257,7 +263,8 @@ __global__ void __launch_bounds__(256) k_hx_levels12(int n1, int n2, int nvec, c
     const T sh = shifts ? shifts[v] : shift0, d2 = dep2 ? dep2[i] : (T)1;
 #pragma unroll
     for (int u = 0; u < PF2; u++) load2(ks + KSPL * u, qa[u], qb[u]);
-    acc_t acc = acc_t{0, 0, 0, 0}, acc2 = acc_t{0, 0, 0, 0};
+    acc_t acc = acc_t{0, 0, 0, 0}, acs = acc_t{0, 0, 0, 0};
+    acc_t &acc2 = ONE ? acc : acs;   // ONE: no DEP, one chain of sums
     const int nch = (n1 + LV_KC - 1) / LV_KC;
     stage_x(0, st[0], sx[0]);
     // chunk ch from its LDS buffer, while chunk ch + 2 loads into the registers that staged it
@@ -270,9 +277,10 @@ __global__ void __launch_bounds__(256) k_hx_levels12(int n1, int n2, int nvec, c
 #pragma unroll
         for (int u = 0; u < GC; u++) {
             constexpr int H0 = decltype(hslot)::value;
+            if (16 * (g0 + KSPL * u) < n1)   // uniform
 #pragma unroll
-            for (int w = 0; w < 4; w++)
-                acc = M::run(sc[16 * KSPL * u + 4 * w], hb[(H0 + u) % PF][w], acc);
+                for (int w = 0; w < 4; w++)
+                    acc = M::run(sc[16 * KSPL * u + 4 * w], hb[(H0 + u) % PF][w], acc);
             load_h(g0 + KSPL * (u + PF), hb[(H0 + u) % PF]);
         }
         stage_x(LV_KC * (ch + 1), next, other);
@@ -305,8 +313,9 @@ __global__ void __launch_bounds__(256) k_hx_levels12(int n1, int n2, int nvec, c
 #pragma unroll
                 for (int w = 0; w < 4; w++) acc2 = M::run(qa[u][w], qb[u][w], acc2);
     }
+    if constexpr (!ONE)
 #pragma unroll
-    for (int q = 0; q < 4; q++) acc[q] += d2 * acc2[q];
+        for (int q = 0; q < 4; q++) acc[q] += d2 * acc2[q];
     if constexpr (KSPL > 1) {
         T *red = sx[0];
         __syncthreads();   // the last chunk is read
@@ -330,19 +339,23 @@ __global__ void __launch_bounds__(256) k_hx_levels12(int n1, int n2, int nvec, c
 // FP64, us with 1 / 2 / 4 waves: n1 = 400, n2 = 96 (150 tiles a vector): 1 vector 11.7 /
 // 8.0 / 7.4, 2 vectors 11.8 / 8.0 / 9.4, 4 vectors 12.0 / 12.2 / 12.2; n1 = 1000,
 // n2 = 64 (252 tiles): 1 vector 20 / 13 / 10, 8 vectors 34 / 39 / 53.
-template <typename T, typename S>
+template <typename T, typename S, bool ONE>
 static void launch_levels12(int n1, int n2, int nplane, int nvec, const T *h1, const T *h2, const T *dep2,
                             const T *res, const T *shifts, T shift0, const S *x, long ldx, S *y, long ldy,
                             const int *active, hipStream_t s)
 {
     const int nti = (n1 + 15) / 16, ntc = (n2 + 15) / 16;
     const long simds = 4L * g_num_cu, tiles = (long)nti * ntc * nplane * nvec;
-#define LV(K, TI, TC)                                                                                           \
-    hipLaunchKernelGGL((k_hx_levels12<T, S, K>), dim3((nti + TI - 1) / TI, (ntc + TC - 1) / TC, nplane *nvec), \
+#define LV(K, TI, TC)                                                                                                \
+    hipLaunchKernelGGL((k_hx_levels12<T, S, K, ONE>), dim3((nti + TI - 1) / TI, (ntc + TC - 1) / TC, nplane *nvec), \
                        dim3(256), 0, s, n1, n2, nvec, h1, h2, dep2, res, shifts, shift0, x, ldx, y, ldy, active)
-    if (4 * tiles <= simds) LV(4, 1, 1);
-    else if (2 * tiles <= simds) LV(2, 2, 1);
-    else LV(1, 2, 2);
+    if constexpr (ONE) {
+        LV(1, 2, 2);
+    } else {
+        if (4 * tiles <= simds) LV(4, 1, 1);
+        else if (2 * tiles <= simds) LV(2, 2, 1);
+        else LV(1, 2, 2);
+    }
 #undef LV
 }
 
@@ -374,8 +387,7 @@ static int hx_generic(scalit_ctx *c, const T *res, const T *shifts, T shift0, in
     int l = 0;
     const Level *L = c->lv;
     if (c->sF >= 2 + (c->ndvr ? 1 : 0) && levels12_fits(L[0].n, L[1].n, L[1].blk, nvec, sizeof(T))) {
-        launch_levels12<T, S>(L[0].n, L[1].n, L[1].blk, nvec, h[0], h[1], dep[1], res, shifts, shift0, x, ldx, y,
-                              ldy, active, s);
+        launch_levels12<T, S, false>(L[0].n, L[1].n, L[1].blk, nvec, h[0], h[1], dep[1], res, shifts, shift0, x, ldx, y, ldy, active, s);
         l = 2;
     } else {
         hipLaunchKernelGGL((k_diag_init<T, S>), g, dim3(th), 0, s, c->N, res, shifts, shift0, x, ldx, y, ldy, active);
@@ -709,7 +721,15 @@ struct VarA {
     int waves, rb, cb;
 };
 static const VarA kVarA[] = {{4, 1, 1}, {4, 3, 2}, {8, 3, 1}, {8, 2, 2}, {8, 1, 2}, {4, 2, 2}, {12, 2, 1}, {12, 1, 2}};
-constexpr int NVA = sizeof(kVarA) / sizeof(kVarA[0]);
+constexpr int NVS = sizeof(kVarA) / sizeof(kVarA[0]);
+// two more, with the same results to the last bit: the pass tile by tile without
+// slabs in LDS (k_hx_levels12), and with mode 3 in it (k_hx_tile3, no pass B).
+// us of the whole operator with slabs / tiles / mode 3 in the tiles, FP64: 24x32x24, 1
+// vector 16.5 / 10.1 / 5.4 (the slab pass is bound by its staging); 37x50x41 30.7 /
+// 14.7 / 10.0; 64x96x80 28.4 / 22.0 / 37, 16 vectors 95 / 159 / -; 128x128x96 (T1 and
+// T2 do not fit beside the slab) 84 / 52 / -, 4 vectors in FP32 106 / 73 / -.
+constexpr int VA_TILES = NVS, VA_FUSED = NVS + 1;
+constexpr int NVA = NVS + 2;
 constexpr int NVB = 3;   // pass B: 4, 8 or 12 waves per workgroup
 
 template <typename T, typename S, bool TL, int W, int RB, int CB>
@@ -763,8 +783,143 @@ static void pass_a(scalit_ctx *c, int va, const T *t1, const T *t2, const T *res
     const bool tl = modes12_lds<T>(n1, n2, true) <= LDS_MAX;
     const size_t lds = modes12_lds<T>(n1, n2, tl);
     dim3 ga(n3 * nvec);
-    if (tl) launch_a<T, S, true>(va, ga, lds, s, n1, n2, n3, nvec, t1, t2, res, sh, sh0, x, ldx, y, ldy, act);
+    if (va >= NVS)
+        launch_levels12<T, S, true>(n1, n2, n3, nvec, t1, t2, nullptr, res, sh, sh0, x, ldx, y, ldy, act, s);
+    else if (tl) launch_a<T, S, true>(va, ga, lds, s, n1, n2, n3, nvec, t1, t2, res, sh, sh0, x, ldx, y, ldy, act);
     else launch_a<T, S, false>(va, ga, lds, s, n1, n2, n3, nvec, t1, t2, res, sh, sh0, x, ldx, y, ldy, act);
+}
+
+// The whole 3-level operator in one launch, for small ones: a workgroup per
+// 16 x 16 tile of a plane (theta point b) and vector.  Wave 0 forms the sums of levels
+// 1 and 2 on MFMA as k_hx_levels12 does; each wave forms mode 3 of a quarter of
+// the tile's points on the vector units, reading those points in every plane
+// (n3 times the reads of the mode-3 pass, from L2, instead of that pass's launch and
+// its read and write of Y).  The additions are in the order of the two passes
+// (bit for bit their results).  Bound by latency: TF3_J planes of a point and four
+// groups of each sum's operands are in flight.
+constexpr int TF3_J = 12;
+template <typename T, typename S>
+__global__ void __launch_bounds__(256) k_hx_tile3(int n1, int n2, int n3, int nvec, const T *__restrict__ h1,
+                                                  const T *__restrict__ h2, const T *__restrict__ h3,
+                                                  const T *__restrict__ dep, const T *__restrict__ res,
+                                                  const T *__restrict__ shifts, T shift0, const S *__restrict__ x,
+                                                  long ldx, S *__restrict__ y, long ldy, const int *__restrict__ active)
+{
+    using M = Mfma<T>;
+    using acc_t = typename M::acc_t;
+    constexpr int PF = 4, ST = (int)sizeof(T), SS = (int)sizeof(S);
+    extern __shared__ char smem_raw[];
+    __shared__ T red[256];
+    T *sx = (T *)smem_raw;   // X(k, c) of the tile's columns at k + lds c, zero past n1
+    const int v = (int)(blockIdx.z % (unsigned)nvec), b = (int)(blockIdx.z / (unsigned)nvec);
+    if (!vec_active(active, v)) return;   // the same for the whole workgroup
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 15, lk = lane >> 4;
+    const int i0 = (int)blockIdx.x * 16, c0 = (int)blockIdx.y * 16;
+    const int P = n1 * n2, n1p = rup16(n1), lds = n1p + 1;
+    const S *xv = x + (long)v * ldx;
+    const int i = min(i0 + lr, n1 - 1), ca = min(c0 + lr, n2 - 1);
+    // loads past the end return zero
+    const auto rv = buf_rsrc(xv, (long)P * n3 * SS), rp = buf_rsrc(xv + (long)P * b, (long)P * SS);
+    const auto rh1 = buf_rsrc(h1, (long)n1 * n1 * ST), rh2 = buf_rsrc(h2, (long)n2 * n2 * ST),
+               rr = buf_rsrc(res + (long)P * b, (long)P * ST), rd = buf_rsrc(dep, (long)P * ST);
+    // this lane's output point: row `wave` of the accumulators
+    const int o = i + n1 * (c0 + M::row(lk, wave));
+    T xj[TF3_J];
+    auto load3 = [&](int j0) {
+#pragma unroll
+        for (int u = 0; u < TF3_J; u++) xj[u] = buf_ld<T, S>(rv, (o + P * min(j0 + u, n3 - 1)) * SS, 0);
+    };
+    // wave 0: A(c,k) = X(k,c) from LDS, B(k,i) = H1(i,k); then A(c,j) = H2(c,j), B(j,i) = X(i,j)
+    const int hv = (i + n1 * lk) * ST, gv = (ca + n2 * lk) * ST, yv = (i + n1 * lk) * SS;
+    T hb[PF][4], qa[PF][4], qb[PF][4];
+    auto load1 = [&](int g, int s) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) hb[s][u] = buf_ld<T, T>(rh1, hv + n1 * (16 * g + 4 * u) * ST, 0);
+    };
+    auto load2 = [&](int g, int s) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            qa[s][u] = buf_ld<T, T>(rh2, gv + n2 * (16 * g + 4 * u) * ST, 0);
+            qb[s][u] = buf_ld<T, S>(rp, yv + n1 * (16 * g + 4 * u) * SS, 0);
+        }
+    };
+    for (int e = tid; e < 16 * n1p; e += 256) {
+        const int c = e / n1p, k = e - c * n1p;
+        const T val = buf_ld<T, S>(rp, (k + n1 * (c0 + c)) * SS, 0);
+        sx[k + lds * c] = k < n1 ? val : (T)0;
+    }
+    if (wave == 0) {
+#pragma unroll
+        for (int u = 0; u < PF; u++) load1(u, u);
+#pragma unroll
+        for (int u = 0; u < PF; u++) load2(u, u);
+    }
+    const T vr = buf_ld<T, T>(rr, o * ST, 0), vx = buf_ld<T, S>(rp, o * SS, 0), vd = buf_ld<T, T>(rd, o * ST, 0);
+    load3(0);
+    __syncthreads();
+    if (wave == 0) {
+        acc_t acc = acc_t{0, 0, 0, 0};
+        const T *sc = sx + lds * lr + lk;
+        const int G1 = n1p / 16, G2 = (n2 + 15) / 16;
+        for (int g = 0; g < G1; g += PF) {
+#pragma unroll
+            for (int u = 0; u < PF; u++) {
+                if (g + u < G1)
+#pragma unroll
+                    for (int w = 0; w < 4; w++) acc = M::run(sc[16 * (g + u) + 4 * w], hb[u][w], acc);
+                if (g + PF < G1) load1(g + u + PF, u);
+            }
+        }
+        for (int g = 0; g < G2; g += PF) {
+#pragma unroll
+            for (int u = 0; u < PF; u++) {
+                if (g + u < G2)
+#pragma unroll
+                    for (int w = 0; w < 4; w++) acc = M::run(qa[u][w], qb[u][w], acc);
+                if (g + PF < G2) load2(g + u + PF, u);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) red[64 * q + lane] = acc[q];
+    }
+    T a3 = 0;
+    for (int j0 = 0;;) {
+#pragma unroll
+        for (int u = 0; u < TF3_J; u++)
+            if (j0 + u < n3) a3 += h3[b + (long)n3 * (j0 + u)] * xj[u];   // uniform
+        j0 += TF3_J;
+        if (j0 >= n3) break;
+        load3(j0);
+    }
+    __syncthreads();
+    const T sh = shifts ? shifts[v] : shift0;
+    T out = red[64 * wave + lane] + (vr - sh) * vx;
+    out += vd * a3;
+    // rows past the last c lie past the plane and are dropped
+    const auto ry = buf_rsrc(y + (long)v * ldy + (long)P * b, (long)P * SS);
+    if (i0 + lr < n1) buf_st<T, S>(ry, o * SS, 0, out);
+}
+
+// The rsrc of k_hx_tile3 spans a vector, and its tiles reach 16 rows past it;
+// X of a tile in LDS.
+template <typename T>
+static bool tile3_fits(const scalit_ctx *c, int nvec)
+{
+    const long n1 = c->lv[0].n;
+    return levels12_fits(n1, c->lv[1].n, c->lv[2].n, nvec, sizeof(T)) &&
+           (c->N + 16 * n1) * (long)sizeof(T) < 0x7fffffffL && n1 <= 256;
+}
+
+template <typename T, typename S>
+static void pass_fused(scalit_ctx *c, const T *t1, const T *t2, const T *l2, const T *dep, const T *res, const T *sh,
+                       T sh0, int nvec, const S *x, long ldx, S *y, long ldy, const int *act, hipStream_t s)
+{
+    const int n1 = c->lv[0].n, n2 = c->lv[1].n, n3 = c->lv[2].n;
+    const size_t lds = (size_t)16 * (rup16(n1) + 1) * sizeof(T);
+    hipLaunchKernelGGL((k_hx_tile3<T, S>), dim3((n1 + 15) / 16, (n2 + 15) / 16, n3 *nvec), dim3(256), lds, s, n1, n2,
+                       n3, nvec, t1, t2, l2, dep, res, sh, sh0, x, ldx, y, ldy, act);
 }
 
 // ---------------------------------------------------------------- autotune
@@ -777,6 +932,20 @@ static int env_variant(const char *name)
     return e ? std::atoi(e) : -1;
 }
 
+// the time of three calls of fn on stream s (after two more), 1e30 when a launch failed
+template <typename Fn>
+static float time_calls(hipEvent_t e0, hipEvent_t e1, hipStream_t s, Fn fn)
+{
+    for (int w = 0; w < 2; w++) fn();
+    (void)hipEventRecord(e0, s);
+    for (int w = 0; w < 3; w++) fn();
+    (void)hipEventRecord(e1, s);
+    (void)hipEventSynchronize(e1);
+    float ms = 0;
+    (void)hipEventElapsedTime(&ms, e0, e1);
+    return hipGetLastError() == hipSuccess ? ms : 1e30f;
+}
+
 template <typename T, typename S>
 static TuneEntry *tune(scalit_ctx *c, int prec, const T *t1, const T *t2, const T *l2, const T *dep, const T *res,
                        const T *sh, T sh0, int nvec, const S *x, long ldx, S *y, long ldy, hipStream_t s)
@@ -787,39 +956,46 @@ static TuneEntry *tune(scalit_ctx *c, int prec, const T *t1, const T *t2, const 
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     (void)hipStreamIsCapturing(s, &st);
     const int n1 = c->lv[0].n, n2 = c->lv[1].n, n3 = c->lv[2].n;
-    TuneEntry e{prec, nvec, fa >= 0 && fa < NVA ? fa : 2, fb >= 0 && fb < NVB ? fb : 0};
+    const bool tiles = levels12_fits(n1, n2, n3, nvec, sizeof(T));
+    const bool fuse = l2 && tile3_fits<T>(c, nvec);
+    const int nva = fuse ? NVA : (tiles ? VA_FUSED : NVS);
+    TuneEntry e{prec, nvec, fa >= 0 && fa < nva ? fa : 2, fb >= 0 && fb < NVB ? fb : 0};
     if (st != hipStreamCaptureStatusNone) return nullptr;   // use the defaults, decide later
-    if (fa < 0 || fb < 0) {
+    // up to one tile per SIMD the fused pass is faster than any pair of passes,
+    // so that nothing is timed (FP64, us: 24x32x24 with 4 vectors, 384 tiles, 6.4
+    // against 10.3 for the tile pass and pass B; 37x50x41 with 2 vectors, 984 tiles, 15.8
+    // against 18.1, with 4 vectors 24.0 against 21.9)
+    const long nt = (long)((n1 + 15) / 16) * ((n2 + 15) / 16) * n3 * nvec;
+    if (fuse && fa < 0 && fb < 0 && nt <= 4L * g_num_cu && n3 <= 48) {
+        e.va = VA_FUSED;
+    } else if (fa < 0 || fb < 0) {
         hipEvent_t e0, e1;
         if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) return nullptr;
-        float best = 1e30f;
-        for (int va = 0; va < NVA && fa < 0; va++) {
-            for (int w = 0; w < 2; w++) pass_a<T, S>(c, va, t1, t2, res, sh, sh0, nvec, x, ldx, y, ldy, nullptr, s);
-            (void)hipEventRecord(e0, s);
-            for (int w = 0; w < 3; w++) pass_a<T, S>(c, va, t1, t2, res, sh, sh0, nvec, x, ldx, y, ldy, nullptr, s);
-            (void)hipEventRecord(e1, s);
-            (void)hipEventSynchronize(e1);
-            float ms = 0;
-            (void)hipEventElapsedTime(&ms, e0, e1);
-            if (hipGetLastError() == hipSuccess && ms < best) {
+        float best = 1e30f, best_b = 1e30f;
+        for (int va = 0; va < std::min(nva, VA_FUSED) && fa < 0; va++) {
+            if (va == 1 || va == 5) continue;   // 4 waves of 3x2 or 2x2 tiles: never the fastest at any size tried
+            const float ms = time_calls(e0, e1, s, [&] {
+                pass_a<T, S>(c, va, t1, t2, res, sh, sh0, nvec, x, ldx, y, ldy, nullptr, s);
+            });
+            if (ms < best) {
                 best = ms;
                 e.va = va;
             }
         }
-        best = 1e30f;
         for (int vb = 0; vb < NVB && fb < 0 && l2; vb++) {
-            for (int w = 0; w < 2; w++) launch_b<T, S>(vb, n1, n2, n3, nvec, l2, dep, x, ldx, y, ldy, nullptr, s);
-            (void)hipEventRecord(e0, s);
-            for (int w = 0; w < 3; w++) launch_b<T, S>(vb, n1, n2, n3, nvec, l2, dep, x, ldx, y, ldy, nullptr, s);
-            (void)hipEventRecord(e1, s);
-            (void)hipEventSynchronize(e1);
-            float ms = 0;
-            (void)hipEventElapsedTime(&ms, e0, e1);
-            if (hipGetLastError() == hipSuccess && ms < best) {
-                best = ms;
+            const float ms = time_calls(e0, e1, s, [&] {
+                launch_b<T, S>(vb, n1, n2, n3, nvec, l2, dep, x, ldx, y, ldy, nullptr, s);
+            });
+            if (ms < best_b) {
+                best_b = ms;
                 e.vb = vb;
             }
         }
+        if (fuse && fa < 0 && fb < 0 && nt <= 8L * g_num_cu &&   // past that it is far behind
+            time_calls(e0, e1, s, [&] {
+                pass_fused<T, S>(c, t1, t2, l2, dep, res, sh, sh0, nvec, x, ldx, y, ldy, nullptr, s);
+            }) < best + best_b)
+            e.va = VA_FUSED;
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
     }
@@ -837,6 +1013,11 @@ static int hx_fast3(scalit_ctx *c, int prec, const T *t1, const T *t2, const T *
     const int n1 = c->lv[0].n, n2 = c->lv[1].n, n3 = c->lv[2].n;
     TuneEntry *te = tune<T, S>(c, prec, t1, t2, l2, dep, res, shifts, shift0, nvec, x, ldx, y, ldy, s);
     const int va = te ? te->va : 2, vb = te ? te->vb : 0;
+    if (va == VA_FUSED && l2) {
+        pass_fused<T, S>(c, t1, t2, l2, dep, res, shifts, shift0, nvec, x, ldx, y, ldy, active, s);
+        HIP_TRY(hipGetLastError());
+        return SCALIT_OK;
+    }
     // modes 1+2 and the diagonal write Y, then mode 3 adds to it
     pass_a<T, S>(c, va, t1, t2, res, shifts, shift0, nvec, x, ldx, y, ldy, active, s);
     if (outh) launch_h3x<T, S>(n1 * n2, n3, nvec, outh, trans_outh, x, ldx, y, ldy, active, s);

@@ -109,3 +109,27 @@ def test_generic_strided_vectors():
         assert (o[1 + v * ld + n:1 + (v + 1) * ld] == 5.0).all()
     assert o[0] == 5.0
     ctx.close()
+
+
+@pytest.mark.parametrize("va", [8, 9])
+@pytest.mark.parametrize("sN,nvec", [((5, 3, 2), 1), ((16, 16, 1), 2), ((17, 33, 7), 3), ((24, 32, 24), 1),
+                                     ((30, 20, 33), 4), ((20, 18, 50), 16), ((70, 40, 9), 2)])
+def test_three_levels_by_tiles(monkeypatch, sN, nvec, va):
+    """The 3-level operator's tile variants: levels 1 and 2 by tiles with the
+    mode-3 pass (8), and mode 3 in the tiles (9); nonsymmetric matrices."""
+    monkeypatch.setenv("SCALIT_HX_VARIANT_A", str(va))
+    monkeypatch.setenv("SCALIT_HX_VARIANT_B", "0")
+    ctx, h0, dep, res = _operator(sN, (2,))
+    ctx.set_shift(0.37)
+    x = P.random_vectors(ctx.N, nvec, 9)
+    xd = ctx.to_device(x)
+    sh = np.linspace(-0.5, 0.5, nvec)
+    assert _rel(ctx.hx(xd, shifts=sh).cpu().numpy(), _reference(h0, dep, res, x, sh)) <= 1e-12
+    assert ctx.hx_variant(L.FP64, nvec)[0] == va
+    dx, _ = ctx.hx_adjoint(xd, xd, L.TA1)
+    assert _rel(dx.cpu().numpy(), _reference(h0, dep, res, x, 0.37, True)) <= 1e-12
+    for dt, tol in ((torch.float32, 2e-6), (torch.bfloat16, 2e-2)):
+        xl = ctx.to_device(x, dt)
+        y = ctx.hx_lp(xl, L.TA1).double().cpu().numpy()
+        assert _rel(y, _reference(h0, dep, res, xl.double().cpu().numpy(), 0.37)) <= tol, dt
+    ctx.close()
