@@ -5,8 +5,8 @@
 //
 // Two paths:
 //  * generic: any number of levels and DEP pattern; the diagonal and levels 1
-//    and 2 in one MFMA pass, then one accumulate-kernel per further level
-//    (thread per output element).
+//    and 2 in one MFMA pass, then one that adds to Y per further level (sizes
+//    past their 32-bit offsets, and one-level operators: thread per output).
 //  * fused 3-level path for sF=3, sDEP=(F,F,T) -- r, R, theta with
 //    DEP(r,R) x L^2_theta -- on FP64 / FP32 MFMA:
 //      pass A, one workgroup per (theta point, vector) slab S(n1 x n2) staged
@@ -395,6 +395,9 @@ static int hx_generic(scalit_ctx *c, const T *res, const T *shifts, T shift0, in
     for (; l < c->sF; l++) {
         if (c->ndvr && l == c->sF - 1)
             launch_h3x<T, S>(L[l].dim, L[l].n, nvec, outh_of<T>(c), transpose, x, ldx, y, ldy, active, s);
+        else if (l > 0 && outer_tiles_fit(L[l].dim, L[l].n, (long)L[l].blk * nvec, sizeof(T)))
+            launch_outer_tiles<T, S, S, true>(L[l].dim, L[l].n, nvec, h[l], 0, dep[l], x, ldx, y, ldy, active, s,
+                                              L[l].blk);
         else
             hipLaunchKernelGGL((k_mode_generic<T, S>), g, dim3(th), 0, s, L[l].dim, L[l].n, L[l].blk, h[l], dep[l],
                                x, ldx, y, ldy, active);
@@ -730,7 +733,7 @@ constexpr int NVS = sizeof(kVarA) / sizeof(kVarA[0]);
 // T2 do not fit beside the slab) 84 / 52 / -, 4 vectors in FP32 106 / 73 / -.
 constexpr int VA_TILES = NVS, VA_FUSED = NVS + 1;
 constexpr int NVA = NVS + 2;
-constexpr int NVB = 3;   // pass B: 4, 8 or 12 waves per workgroup
+constexpr int VB_TILES = 3, NVB = 4;   // pass B: 4, 8 or 12 waves per workgroup, or tile by tile
 
 template <typename T, typename S, bool TL, int W, int RB, int CB>
 static void launch_a1(dim3 g, size_t lds, hipStream_t s, int n1, int n2, int n3, int nvec, const T *t1, const T *t2,
@@ -770,7 +773,8 @@ static void launch_b(int vb, int n1, int n2, int n3, int nvec, const T *l2, cons
                      long ldy, const int *act, hipStream_t s)
 {
     const long P = (long)n1 * n2;
-    if (vb == 0) launch_outer_mode<T, S, S, 4, true>(P, n3, nvec, l2, dep, x, ldx, y, ldy, act, s);
+    if (vb == VB_TILES) launch_outer_tiles<T, S, S, true>(P, n3, nvec, l2, 0, dep, x, ldx, y, ldy, act, s);
+    else if (vb == 0) launch_outer_mode<T, S, S, 4, true>(P, n3, nvec, l2, dep, x, ldx, y, ldy, act, s);
     else if (vb == 1) launch_outer_mode<T, S, S, 8, true>(P, n3, nvec, l2, dep, x, ldx, y, ldy, act, s);
     else launch_outer_mode<T, S, S, 12, true>(P, n3, nvec, l2, dep, x, ldx, y, ldy, act, s);
 }
@@ -959,7 +963,7 @@ static TuneEntry *tune(scalit_ctx *c, int prec, const T *t1, const T *t2, const 
     const bool tiles = levels12_fits(n1, n2, n3, nvec, sizeof(T));
     const bool fuse = l2 && tile3_fits<T>(c, nvec);
     const int nva = fuse ? NVA : (tiles ? VA_FUSED : NVS);
-    TuneEntry e{prec, nvec, fa >= 0 && fa < nva ? fa : 2, fb >= 0 && fb < NVB ? fb : 0};
+    TuneEntry e{prec, nvec, fa >= 0 && fa < nva ? fa : 2, fb >= 0 && fb < (outer_tiles_fit((long)n1 * n2, n3, nvec, sizeof(T)) ? NVB : VB_TILES) ? fb : 0};
     if (st != hipStreamCaptureStatusNone) return nullptr;   // use the defaults, decide later
     // up to one tile per SIMD the fused pass is faster than any pair of passes,
     // so that nothing is timed (FP64, us: 24x32x24 with 4 vectors, 384 tiles, 6.4
@@ -983,6 +987,7 @@ static TuneEntry *tune(scalit_ctx *c, int prec, const T *t1, const T *t2, const 
             }
         }
         for (int vb = 0; vb < NVB && fb < 0 && l2; vb++) {
+            if (vb == VB_TILES && !outer_tiles_fit((long)n1 * n2, n3, nvec, sizeof(T))) continue;
             const float ms = time_calls(e0, e1, s, [&] {
                 launch_b<T, S>(vb, n1, n2, n3, nvec, l2, dep, x, ldx, y, ldy, nullptr, s);
             });

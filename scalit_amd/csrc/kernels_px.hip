@@ -8,7 +8,8 @@
 // contiguous inner index k (NIN = n_1...n_{l-1} values).  k_outer_mode
 // computes it on MFMA with one grid row per block: the block's rotation is
 // staged in LDS, each wave takes 16-point tiles of k (coalesced runs along k)
-// with all of j in registers, as the mode-3 pass of H*X does.
+// with all of j in registers, as the mode-3 pass of H*X does; single vectors and
+// small grids go tile by tile (k_outer_tiles).
 //
 // Level 1 (the innermost, NIN = 1) holds one n1 x n1 rotation per block of
 // all outer indices: VOSB level 1 is N*n1 values, the largest stream of the
@@ -305,24 +306,33 @@ static size_t l1_lds(int n1, bool mf)
     return (ns * (ns + 1) + 2 * wc * (ns + 1) + 256 + ns + 2 * wc) * sizeof(T) + 2 * wc * sizeof(int);
 }
 
-// One rotation level, VTX (trans) or VX: MFMA when the block fits (n <= 128),
-// else one thread per value.  vosbt holds the per-block transposes.
+// One rotation level, VTX (trans) or VX, on MFMA: tile by tile for few tiles
+// and for blocks past 128, else a block's rotation per workgroup; one thread per value
+// past the tiles' offsets.  vosbt holds the per-block transposes.
+//
+// The line between the two by tiles x n, the MFMA work.  Whole P*X in us, staged / by tiles,
+// FP64: 24x32x24 28.2 / 21.0 for one vector and 37.8 / 32.0 for 16 (49 k), 48x64x40
+// 74.6 / 66.5 for 8 (246 k) and 90.8 / 91.9 for 16 (490 k), 64x96x80 103.8 / 83.7 for one (184 k) and
+// 118 / 112 for two (369 k), 80x96x64 191 / 194 for two (369 k); FP32: 48x64x40 70 / 54 for 16 (490 k),
+// 64x96x80 93 / 88 for 4 and 80x96x64 127 / 128 for 4 (740 k).
 template <typename T, typename SI, typename SO>
 static void rotate(const Level &L, const T *vosb, const T *vosbt, bool trans, int nvec, const SI *x, long ldx, SO *y,
                    long ldy, const int *active, hipStream_t s)
 {
     const int nin = L.dim, n = L.n, blk = L.blk;
-    if (n > 128 || blk > 65535 || (size_t)rup16(n) * rup16(n) * sizeof(T) > PX_LDS_MAX) {
-        dim3 g(pgrid((long)nin * n * blk), nvec);
-        hipLaunchKernelGGL((k_rotate_generic<T, SI, SO>), g, dim3(256), 0, s, nin, n, blk, vosb, trans, x, ldx, y, ldy,
-                           active);
-        return;
-    }
+    const T *mats = trans ? vosbt : vosb;
+    const long nz = (long)blk * nvec;
+    const bool staged = n <= 128 && blk <= 65535 && (size_t)rup16(n) * rup16(n) * sizeof(T) <= PX_LDS_MAX;
+    const long few = sizeof(T) == 8 ? 1L << 18 : 1L << 19;
+    if (outer_tiles_fit(nin, n, nz, sizeof(T)) && (!staged || outer_tiles(nin, n, nz) * n <= few))
+        launch_outer_tiles<T, SI, SO, false>(nin, n, nvec, mats, (long)n * n, nullptr, x, ldx, y, ldy, active, s, blk);
+    else if (!staged)
+        hipLaunchKernelGGL((k_rotate_generic<T, SI, SO>), dim3(pgrid((long)nin * n * blk), nvec), dim3(256), 0, s, nin,
+                           n, blk, vosb, trans, x, ldx, y, ldy, active);
     // the persistent outer-mode kernel, one grid row per block: 8 waves per
     // workgroup for batches, 4 for a single vector (fastest measured on the
     // 64x96x80 workload)
-    const T *mats = trans ? vosbt : vosb;
-    if (nvec >= 4)
+    else if (nvec >= 4)
         launch_outer_mode<T, SI, SO, 8, false>(nin, n, nvec, mats, nullptr, x, ldx, y, ldy, active, s, blk);
     else
         launch_outer_mode<T, SI, SO, 4, false>(nin, n, nvec, mats, nullptr, x, ldx, y, ldy, active, s, blk);

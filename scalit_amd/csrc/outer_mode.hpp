@@ -171,6 +171,97 @@ __global__ void __launch_bounds__(64 * WAVES) k_outer_mode(long P, int n, int nv
     }
 }
 
+// The same product tile by tile, for few tiles: one wave per 16 p x 16 i tile,
+// A and X straight into fragments (both walk memory along the lanes) with
+// OT_PF groups of 16 k in flight; loads past the end return zero.  k_outer_mode
+// stages a whole matrix per workgroup and gives a wave all of i, which pays from
+// some thousand tiles on; below, its staging and the long chain per wave are what
+// takes the time (64x96x80, one FP64 vector, the four rotations of a P*X: 52 us
+// against 32).  The additions are in the same order: the
+// same results to the last bit.  Block b's matrix at amat + astride b.
+constexpr int OT_PF = 4;
+template <typename T, typename S, typename SO, bool ACC>
+__global__ void __launch_bounds__(256) k_outer_tiles(int P, int n, int nvec, const T *__restrict__ amat, long astride,
+                                                    const T *__restrict__ dvec, const S *__restrict__ x, long ldx,
+                                                    SO *__restrict__ y, long ldy, const int *active)
+{
+    using M = Mfma<T>;
+    using acc_t = typename M::acc_t;
+    constexpr int ST = (int)sizeof(T), SS = (int)sizeof(S), SY = (int)sizeof(SO);
+    const int v = (int)(blockIdx.z % (unsigned)nvec);
+    const long b = blockIdx.z / (unsigned)nvec;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lr = lane & 15, lk = lane >> 4;
+    const int p0 = ((int)blockIdx.x * 4 + wave) * 16, i0 = (int)blockIdx.y * 16;
+    if (p0 >= P || !vec_active(active, v)) return;
+    const long blk = (long)P * n;
+    const auto rx = buf_rsrc(x + (long)v * ldx + blk * b, blk * SS);
+    const auto ra = buf_rsrc(amat + astride * b, (long)n * n * ST);
+    const auto ry = buf_rsrc(y + (long)v * ldy + blk * b, blk * SY);
+    const int p = min(p0 + lr, P - 1);
+    const int av = (min(i0 + lr, n - 1) + n * lk) * ST, xv = (p + P * lk) * SS;
+    T a[OT_PF][4], bx[OT_PF][4];
+    auto load = [&](int g, int s) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            a[s][u] = buf_ld<T, T>(ra, av + n * (16 * g + 4 * u) * ST, 0);
+            bx[s][u] = buf_ld<T, S>(rx, xv + P * (16 * g + 4 * u) * SS, 0);
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < OT_PF; u++) load(u, u);
+    const int yo = p + P * (i0 + M::row(lk, 0));
+    T yc[4];
+    if constexpr (ACC)
+#pragma unroll
+        for (int q = 0; q < 4; q++) yc[q] = buf_ld<T, SO>(ry, (yo + P * M::row(0, q)) * SY, 0);
+    const T d = dvec ? dvec[p] : (T)1;
+    acc_t acc = acc_t{0, 0, 0, 0};
+    const int G = (n + 15) / 16;
+    int g = 0;
+    for (; g + OT_PF <= G; g += OT_PF) {
+#pragma unroll
+        for (int u = 0; u < OT_PF; u++) {
+#pragma unroll
+            for (int w = 0; w < 4; w++) acc = M::run(a[u][w], bx[u][w], acc);
+            load(g + u + OT_PF, u);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < OT_PF - 1; u++)
+        if (g + u < G)
+#pragma unroll
+            for (int w = 0; w < 4; w++) acc = M::run(a[u][w], bx[u][w], acc);
+    // rows past the last i lie past the block and are dropped
+    if (p0 + lr < P)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            T out = d * acc[q];
+            if constexpr (ACC) out += yc[q];
+            buf_st<T, SO>(ry, (yo + P * M::row(0, q)) * SY, 0, out);
+        }
+}
+
+// 32-bit byte offsets of the loads in flight (fewer than 1,024 indices past the
+// end), the grid's z range
+static inline bool outer_tiles_fit(long P, long n, long nz, size_t item)
+{
+    return (P + 1024) * (n + 1024) * (long)item < 0x7fffffffL && (n + 1024) * (n + 1024) * (long)item < 0x7fffffffL &&
+           nz <= 65535;
+}
+// waves of the tile form
+static inline long outer_tiles(long P, long n, long nz) { return ((P + 15) / 16) * ((n + 15) / 16) * nz; }
+
+template <typename T, typename S, typename SO, bool ACC>
+static void launch_outer_tiles(long P, int n, int nvec, const T *amat, long astride, const T *dvec, const S *x, long ldx,
+                               SO *y, long ldy, const int *active, hipStream_t s, int nblk = 1)
+{
+    hipLaunchKernelGGL((k_outer_tiles<T, S, SO, ACC>),
+                       dim3((unsigned)((P + 63) / 64), (unsigned)((n + 15) / 16), (unsigned)(nblk * nvec)), dim3(256), 0,
+                       s, (int)P, n, nvec, amat, astride, dvec, x, ldx, y, ldy, active);
+}
+
 // Launch with WAVES waves per workgroup and as many workgroups as fit on the
 // device at once (at most one per 16 tiles' worth of waves).
 template <typename T, typename S, typename SO, int WAVES, int NR, bool ACC>

@@ -31,6 +31,8 @@ SHAPES = [
     ((31, 5, 4), (), 2),
     ((20, 18, 7), (1, 2), 9),
     ((6, 5, 4, 7), (1, 3), 3),
+    ((4, 3, 17, 5), (2, 3), 2),
+    ((3, 2, 200), (2,), 3),
 ]
 
 
@@ -111,25 +113,60 @@ def test_generic_strided_vectors():
     ctx.close()
 
 
-@pytest.mark.parametrize("va", [8, 9])
+@pytest.mark.parametrize("va,vb", [(8, 3), (9, 0), (2, 3)])
 @pytest.mark.parametrize("sN,nvec", [((5, 3, 2), 1), ((16, 16, 1), 2), ((17, 33, 7), 3), ((24, 32, 24), 1),
                                      ((30, 20, 33), 4), ((20, 18, 50), 16), ((70, 40, 9), 2)])
-def test_three_levels_by_tiles(monkeypatch, sN, nvec, va):
-    """The 3-level operator's tile variants: levels 1 and 2 by tiles with the
-    mode-3 pass (8), and mode 3 in the tiles (9); nonsymmetric matrices."""
+def test_three_levels_by_tiles(monkeypatch, sN, nvec, va, vb):
+    """The 3-level operator's tile variants: levels 1 and 2 by tiles (8), mode 3
+    in the tiles (9), the mode-3 pass by tiles (3); nonsymmetric matrices."""
     monkeypatch.setenv("SCALIT_HX_VARIANT_A", str(va))
-    monkeypatch.setenv("SCALIT_HX_VARIANT_B", "0")
+    monkeypatch.setenv("SCALIT_HX_VARIANT_B", str(vb))
     ctx, h0, dep, res = _operator(sN, (2,))
     ctx.set_shift(0.37)
     x = P.random_vectors(ctx.N, nvec, 9)
     xd = ctx.to_device(x)
     sh = np.linspace(-0.5, 0.5, nvec)
     assert _rel(ctx.hx(xd, shifts=sh).cpu().numpy(), _reference(h0, dep, res, x, sh)) <= 1e-12
-    assert ctx.hx_variant(L.FP64, nvec)[0] == va
+    assert ctx.hx_variant(L.FP64, nvec) == (va, vb)
     dx, _ = ctx.hx_adjoint(xd, xd, L.TA1)
     assert _rel(dx.cpu().numpy(), _reference(h0, dep, res, x, 0.37, True)) <= 1e-12
     for dt, tol in ((torch.float32, 2e-6), (torch.bfloat16, 2e-2)):
         xl = ctx.to_device(x, dt)
         y = ctx.hx_lp(xl, L.TA1).double().cpu().numpy()
         assert _rel(y, _reference(h0, dep, res, xl.double().cpu().numpy(), 0.37)) <= tol, dt
+    ctx.close()
+
+
+@pytest.mark.parametrize("sN,nvec", [((5, 3, 2), 1), ((16, 17, 16), 2), ((24, 32, 24), 3), ((7, 130, 3), 2),
+                                     ((70, 40, 9), 1)])
+def test_rotations_by_tiles(sN, nvec):
+    """P*X with the level >= 2 rotations tile by tile (also past 128 points), on
+    seeded orthogonal rotations, against dense products; FP64 1e-12, FP32 1e-5
+    (the shift lies below every EIG0, so the divide amplifies nothing)."""
+    g = P.rng(4)
+    ctx = Context(sN, [False] * len(sN))
+    n = ctx.N
+    vosb = []
+    for l, m in enumerate(sN):
+        q = np.linalg.qr(g.standard_normal((ctx.blk[l], m, m)))[0]
+        vosb.append(q.transpose(0, 2, 1).reshape(-1))   # column-major blocks
+    eig0 = g.uniform(1.0, 2.0, size=n)
+    ctx.set_precond(vosb, eig0)
+    ctx.set_res(np.zeros(n))
+    ctx.set_shift(0.5)
+    x = P.random_vectors(n, nvec, 12)
+
+    def rot(z, l, trans):
+        q = vosb[l].reshape(ctx.blk[l], sN[l], sN[l]).transpose(0, 2, 1)
+        z = z.reshape(nvec, ctx.blk[l], sN[l], ctx.dim[l])
+        return np.einsum("bji,vbjk->vbik" if trans else "bij,vbjk->vbik", q, z).reshape(nvec, n)
+
+    z = x
+    for l in (2, 1, 0):
+        z = rot(z, l, True)
+    z = z / (eig0 - 0.5)
+    for l in (0, 1, 2):
+        z = rot(z, l, False)
+    assert _rel(ctx.px(ctx.to_device(x)).cpu().numpy(), z) <= 1e-12
+    assert _rel(ctx.px_lp(ctx.to_device(x, torch.float32)).double().cpu().numpy(), z) <= 1e-5
     ctx.close()
