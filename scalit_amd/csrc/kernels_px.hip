@@ -74,9 +74,12 @@ __global__ void k_rotate_generic(int nin, int nout, int blk, const T *__restrict
 // ns = n1 rounded up to 16, else ns = n1), W and Z ((ns+1) x WC each; W holds
 // Y after the MF product), partial sums (256), EIG0 of the block (ns), and
 // the shifts and activity of the first chunk of vectors and of the current
-// later one (2 WC each).  BIG (n1 > 64): the part of a block beyond the
-// registers is loaded while it is staged.
-template <typename T, typename S, typename SO, bool MF, bool BIG>
+// later one (2 WC each).  NP: the block size the registers of the prefetch hold (64,
+// 80, 96 or 112: (NP / 16)^2 rotation values and NP / 16 first-chunk values per thread); with
+// larger blocks (n1 > 112, VALU) the rest is loaded while it is staged.  Prefetching
+// a whole block of 80 points instead of its first 4,096 values took this kernel from 90 to 79 us at 80x96x64 with 16
+// FP32 vectors, and the whole P*X of one FP64 vector there from 153 to 112 us.
+template <typename T, typename S, typename SO, bool MF, int NP>
 __global__ void __launch_bounds__(256) k_px_l1(int n1, int nblk, int nvec, const T *__restrict__ vosb,
                                                const T *__restrict__ eig0, const T *__restrict__ shifts, T shift0,
                                                int nosb, T de, T beta, const S *__restrict__ x, long ldx,
@@ -85,8 +88,9 @@ __global__ void __launch_bounds__(256) k_px_l1(int n1, int nblk, int nvec, const
     using M = Mfma<T>;
     using acc_t = typename M::acc_t;
     constexpr int WC = MF ? 16 : 8;   // vectors per chunk
-    constexpr int PV = 16;            // rotation values per thread
-    constexpr int PY = MF ? 4 : 2;    // first-chunk values per thread
+    constexpr int PV = (NP / 16) * (NP / 16);      // rotation values per thread
+    constexpr int PY = (NP * WC + 255) / 256;      // first-chunk values per thread
+    constexpr bool BIG = NP == 112 && !MF;         // blocks past the registers
     extern __shared__ char smem_raw[];
     const int ns = MF ? rup16(n1) : n1;
     const int ldv = ns + 1;
@@ -100,6 +104,7 @@ __global__ void __launch_bounds__(256) k_px_l1(int n1, int nblk, int nvec, const
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 15, lk = lane >> 4;
+    const float r1 = 1.0f / (float)n1, rs = 1.0f / (float)ns;   // e / n1 and e / ns (fdiv_small)
     const int G = gridDim.x;
     const int nvv = n1 * n1;
     const int nw = ns * WC;   // values of one chunk of vectors
@@ -122,35 +127,41 @@ __global__ void __launch_bounds__(256) k_px_l1(int n1, int nblk, int nvec, const
         const bool live = bb < nblk;
         const long b0 = min(bb, nblk - 1);
         const T *vb = vosb + b0 * nvv;
+        int t0 = tid;   // opaque past 64 points: the offsets are not kept in registers from block to block
+        if constexpr (NP > 64) asm volatile("" : "+v"(t0));
 #pragma unroll
-        for (int u = 0; u < PV; u++) pv[u] = vb[live ? min(tid + 256 * u, nvv - 1) : 0];
+        for (int u = 0; u < PV; u++) pv[u] = vb[live ? min(t0 + 256 * u, nvv - 1) : 0];
 #pragma unroll
         for (int u = 0; u < PY; u++) {
-            const int e = tid + 256 * u;
-            const int j = live ? min(e % ns, n1 - 1) : 0, v = live ? min(e / ns, nvec - 1) : 0;
+            const int e = t0 + 256 * u;
+            const int c = fdiv_small(e, rs);
+            const int j = live ? min(e - ns * c, n1 - 1) : 0, v = live ? min(c, nvec - 1) : 0;
             py[u] = ld_cvt<T, S>(x + (long)v * ldx + b0 * n1, j);
         }
         pe = eig0[b0 * n1 + (live ? min(tid, n1 - 1) : 0)];
     };
     auto stage = [&](int bb) {
+        int t0 = tid;
+        if constexpr (NP > 64) asm volatile("" : "+v"(t0));
 #pragma unroll
         for (int u = 0; u < PV; u++) {
-            const int e = tid + 256 * u;
-            if (e < nvv) sV[(e % n1) + ldv * (e / n1)] = pv[u];
+            const int e = t0 + 256 * u;
+            const int c = fdiv_small(e, r1);
+            if (e < nvv) sV[e + (ldv - n1) * c] = pv[u];
         }
         if constexpr (BIG)
-            for (int e = tid + 256 * PV; e < nvv; e += 256) sV[(e % n1) + ldv * (e / n1)] = vosb[(long)bb * nvv + e];
+            for (int e = tid + 256 * PV; e < nvv; e += 256) sV[e + (ldv - n1) * fdiv_small(e, r1)] = vosb[(long)bb * nvv + e];
 #pragma unroll
         for (int u = 0; u < PY; u++) {
-            const int e = tid + 256 * u;
+            const int e = t0 + 256 * u;
             if (e < nw) {
-                const int j = e % ns, c = e / ns;
+                const int c = fdiv_small(e, rs), j = e - ns * c;
                 sW[j + ldv * c] = (j < n1 && sAct[c]) ? py[u] : (T)0;
             }
         }
         if constexpr (BIG)
             for (int e = tid + 256 * PY; e < nw; e += 256) {
-                const int j = e % ns, c = e / ns;
+                const int c = fdiv_small(e, rs), j = e - ns * c;
                 sW[j + ldv * c] = (j < n1 && sAct[c]) ? ld_cvt<T, S>(x + (long)c * ldx + (long)bb * n1, j) : (T)0;
             }
         if (tid < ns) sE[tid] = tid < n1 ? pe : (T)0;
@@ -164,7 +175,7 @@ __global__ void __launch_bounds__(256) k_px_l1(int n1, int nblk, int nvec, const
                 vec_info(v0, 1);
                 __syncthreads();
                 for (int e = tid; e < nw; e += 256) {
-                    const int j = e % ns, c = e / ns;
+                    const int c = fdiv_small(e, rs), j = e - ns * c;
                     sW[j + ldv * c] = (j < n1 && sAct[WC + c])
                                           ? ld_cvt<T, S>(x + (long)(v0 + c) * ldx + (long)bb * n1, j)
                                           : (T)0;
@@ -217,7 +228,7 @@ __global__ void __launch_bounds__(256) k_px_l1(int n1, int nblk, int nvec, const
                 }
                 __syncthreads();
                 for (int e = tid; e < n1 * WC; e += 256) {
-                    const int i = e % n1, c = e / n1;
+                    const int c = fdiv_small(e, r1), i = e - n1 * c;
                     if (act[c]) st_cvt<T, SO>(y + (long)(v0 + c) * ldy + (long)bb * n1, i, sW[i + ldv * c]);
                 }
             } else {
@@ -230,7 +241,7 @@ __global__ void __launch_bounds__(256) k_px_l1(int n1, int nblk, int nvec, const
                 const int sl = (n1 + np - 1) / np;
                 if (np == 1) {
                     for (int e = tid; e < no; e += 256) {
-                        const int i = e % n1, c = e / n1;
+                        const int c = fdiv_small(e, r1), i = e - n1 * c;
                         T acc = 0;
 #pragma unroll 8
                         for (int j = 0; j < n1; j++) acc += sV[j + ldv * i] * sW[j + ldv * c];
@@ -238,7 +249,7 @@ __global__ void __launch_bounds__(256) k_px_l1(int n1, int nblk, int nvec, const
                     }
                     __syncthreads();
                     for (int e = tid; e < no; e += 256) {
-                        const int i = e % n1, c = e / n1;
+                        const int c = fdiv_small(e, r1), i = e - n1 * c;
                         if (!act[c]) continue;
                         T acc = 0;
 #pragma unroll 8
@@ -246,8 +257,8 @@ __global__ void __launch_bounds__(256) k_px_l1(int n1, int nblk, int nvec, const
                         st_cvt<T, SO>(y + (long)(v0 + c) * ldy + (long)bb * n1, i, acc);
                     }
                 } else {
-                    const int o = tid % no, q = tid / no;   // output, slice
-                    const int i = o % n1, c = o / n1;
+                    const int q = fdiv_small(tid, 1.0f / (float)no), o = tid - no * q;   // slice, output
+                    const int c = fdiv_small(o, r1), i = o - n1 * c;
                     const int j0 = q * sl, j1 = min(n1, j0 + sl);
                     if (q < np) {
                         T acc = 0;
@@ -323,7 +334,7 @@ static void rotate(const Level &L, const T *vosb, const T *vosbt, bool trans, in
     const T *mats = trans ? vosbt : vosb;
     const long nz = (long)blk * nvec;
     const bool staged = n <= 128 && blk <= 65535 && (size_t)rup16(n) * rup16(n) * sizeof(T) <= PX_LDS_MAX;
-    const long few = sizeof(T) == 8 ? 1L << 18 : 1L << 19;
+    const long few = sizeof(T) == 8 ? 1L << 18 : 3L << 18;
     if (outer_tiles_fit(nin, n, nz, sizeof(T)) && (!staged || outer_tiles(nin, n, nz) * n <= few))
         launch_outer_tiles<T, SI, SO, false>(nin, n, nvec, mats, (long)n * n, nullptr, x, ldx, y, ldy, active, s, blk);
     else if (!staged)
@@ -338,37 +349,43 @@ static void rotate(const Level &L, const T *vosb, const T *vosbt, bool trans, in
         launch_outer_mode<T, SI, SO, 4, false>(nin, n, nvec, mats, nullptr, x, ldx, y, ldy, active, s, blk);
 }
 
-template <typename T, typename SI, typename SO, bool MF, bool BIG>
+template <typename T, typename SI, typename SO, bool MF, int NP>
 static void launch_l1(int n1, int nb, const T *vosb, const T *eig0, const T *shifts, T shift0, int nosb, T de, T beta,
                       int nvec, const SI *x, long ldx, SO *y, long ldy, const int *active, hipStream_t s)
 {
     // persistent: as many workgroups as are resident at once (per LDS size)
     const size_t lds = l1_lds<T>(n1, MF);
-    const int per_cu = resident_per_cu((const void *)k_px_l1<T, SI, SO, MF, BIG>, 256, lds);
+    const int per_cu = resident_per_cu((const void *)k_px_l1<T, SI, SO, MF, NP>, 256, lds);
     const int G = std::min(nb, g_num_cu * per_cu);
-    hipLaunchKernelGGL((k_px_l1<T, SI, SO, MF, BIG>), dim3(G), dim3(256), lds, s, n1, nb, nvec, vosb, eig0, shifts, shift0,
+    hipLaunchKernelGGL((k_px_l1<T, SI, SO, MF, NP>), dim3(G), dim3(256), lds, s, n1, nb, nvec, vosb, eig0, shifts, shift0,
                        nosb, de, beta, x, ldx, y, ldy, active);
 }
 
-// Level 1: MFMA for batches of 8 and more, VALU otherwise.
+// Level 1: MFMA for batches of 8 and more, and where the VALU form has more
+// outputs than threads; VALU otherwise.  Whole P*X in FP64, us, VALU / MFMA: 48x64x40 56.0 /
+// 57.2 for 5 vectors (240 outputs), 63.2 / 59.3 for 6; 64x96x80 151 / 153 for 4 (256),
+// 176 / 159 for 5; 80x96x64 165 / 192 for 3 (240), 217 / 199 for 4; 96x64x40 124 / 139
+// for 2 (192), 188 / 147 for 3.
 template <typename T, typename SI, typename SO>
 static void level1(const Level &L, const T *vosb, const T *eig0, const T *shifts, T shift0, int nosb, T de, T beta,
                    int nvec, const SI *x, long ldx, SO *y, long ldy, const int *active, hipStream_t s)
 {
     const int n1 = L.n, nb = L.blk;
-    const bool mf = nvec >= 8 && n1 <= 112 && l1_lds<T>(n1, true) <= PX_LDS_MAX;
-    if (mf && n1 <= 64)
-        launch_l1<T, SI, SO, true, false>(n1, nb, vosb, eig0, shifts, shift0, nosb, de, beta, nvec, x, ldx, y, ldy,
-                                          active, s);
-    else if (mf)
-        launch_l1<T, SI, SO, true, true>(n1, nb, vosb, eig0, shifts, shift0, nosb, de, beta, nvec, x, ldx, y, ldy,
-                                         active, s);
-    else if (n1 <= 64)
-        launch_l1<T, SI, SO, false, false>(n1, nb, vosb, eig0, shifts, shift0, nosb, de, beta, nvec, x, ldx, y, ldy,
-                                           active, s);
-    else
-        launch_l1<T, SI, SO, false, true>(n1, nb, vosb, eig0, shifts, shift0, nosb, de, beta, nvec, x, ldx, y, ldy,
-                                          active, s);
+    const bool mf = (nvec >= 8 || n1 * nvec > 256) && n1 <= 112 && l1_lds<T>(n1, true) <= PX_LDS_MAX;
+#define L1(M, N) \
+    launch_l1<T, SI, SO, M, N>(n1, nb, vosb, eig0, shifts, shift0, nosb, de, beta, nvec, x, ldx, y, ldy, active, s)
+    if (mf) {
+        if (n1 <= 64) L1(true, 64);
+        else if (n1 <= 80) L1(true, 80);
+        else if (n1 <= 96) L1(true, 96);
+        else L1(true, 112);
+    } else {
+        if (n1 <= 64) L1(false, 64);
+        else if (n1 <= 80) L1(false, 80);
+        else if (n1 <= 96) L1(false, 96);
+        else L1(false, 112);
+    }
+#undef L1
 }
 
 // Level-1 rotations too large for the fused kernel's LDS (n1 > 256: the
