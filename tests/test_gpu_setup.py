@@ -76,6 +76,28 @@ def test_setup_other_levels(sN, deps):
     _check(sN, h0, dep, g.standard_normal(dim))
 
 
+@pytest.mark.parametrize("grid", [(24, 32, 24), (16, 48, 30)])
+def test_setup_rotations_orthogonal(grid):
+    """V^T V - 1 over all blocks of a level, in the root mean square: what the
+    oracle's cos, sin and updates leave, and a quarter more for the scatter of a
+    level of a few hundred entries and for roundings in another order."""
+    prob = P.config_problem("hx_bench", 1, grid)
+    vo, _ = O.Operator(prob.sN, prob.h0, prob.res, prob.dep).diag(1000, 1e-5)
+    ctx = Context.from_problem(prob)
+    ctx.block_diag(1000, 1e-5)
+    v, _ = ctx.get_precond()
+    ctx.close()
+
+    def defect(v, n):
+        w = np.asarray(v).reshape(-1, n, n)   # rows: the columns of V
+        return float(np.sqrt(np.mean((w @ w.transpose(0, 2, 1) - np.eye(n)) ** 2)))
+
+    for l, n in enumerate(grid):
+        d, ref = defect(v[l], n), defect(vo[l], n)
+        print(grid, "level", l + 1, d, "oracle", ref, flush=True)
+        assert d <= 1.25 * ref
+
+
 @pytest.mark.parametrize("bjmax,bjtol", [(0, 1e-5), (1, 1e-5), (3, 0.0), (1000, 1e-9)])
 def test_setup_stopping(bjmax, bjtol):
     """No sweep, one, a fixed count (tolerance 0), and a tight tolerance."""
