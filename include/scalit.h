@@ -130,7 +130,9 @@ int scalit_set_qmr_persistent(scalit_ctx *ctx, int on);
 
 /* OSB set-up on the GPU: myDiag (src/iterate/module/osb.diag.h:53-151) with
  * HosbDiag/MJACOBI (src/iterate/libiterate/diag/hosbdiag.f90:5-75,
- * jacobi.f90:2-83).  Leaves VOSB and EIG0 resident. */
+ * jacobi.f90:2-83).  Leaves VOSB and EIG0 resident.  The fast form takes
+ * levels whose H0 is symmetric to rounding; of any other H0 it uses what
+ * MJACOBI reads (the columns of each pair as they are rotated, then mirrored). */
 int scalit_block_diag(scalit_ctx *ctx, int bjmax, double bjtol);
 /* Load / fetch VOSB and EIG0 (host arrays, the sVOSB<0 / >0 file modes,
  * src/iterate/module/osb.progDiag.h:6-25): vosb[l] holds myBlk(l)*n_l^2. */

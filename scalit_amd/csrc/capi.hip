@@ -273,6 +273,13 @@ int scalit_set_h0(scalit_ctx *c, int level, const double *h0)
     std::vector<double> t((size_t)n * n);
     for (int i = 0; i < n; i++)
         for (int j = 0; j < n; j++) t[i + (size_t)n * j] = h0[j + (size_t)n * i];
+    // symmetric to the rounding of a product that forms H0 (W^T T W of a PO-DVR is
+    // not symmetric in the last places); a NaN counts as not symmetric
+    double big = 0.0;
+    for (size_t e = 0; e < t.size(); e++) big = std::max(big, std::fabs(h0[e]));
+    const double tol = n * 2.220446049250313e-16 * big;
+    L.h0_sym = true;
+    for (size_t e = 0; e < t.size(); e++) L.h0_sym = L.h0_sym && std::fabs(h0[e] - t[e]) <= tol;
     HIP_TRY(hipMemcpy(L.h0.p, h0, sizeof(double) * n * n, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(L.h0t.p, t.data(), sizeof(double) * n * n, hipMemcpyHostToDevice));
     L.has_h0 = true;

@@ -9,8 +9,9 @@
 //   |d offdiag| <= tol * initial or BJMAX sweeps (hosbdiag.f90:5-75);
 //   VOSB accumulates the rotations (vupdate.f90:21-36), EIG0 <- diag(HOSB).
 //
-// Real separable levels of up to 128 points: kernels_jacobi.hip.  The others
-// (complex level matrices, the dense sNDVR layer, larger levels) here:
+// Real separable levels of up to 128 points with a symmetric H0:
+// kernels_jacobi.hip.  The others (complex level matrices, the dense sNDVR layer,
+// larger levels, an H0 that is not symmetric, of which MJACOBI reads a part) here:
 //
 // Level 1 (NDK = 1): one wave per block runs the whole Jacobi in LDS.
 // Levels with NDK > 1: one launch per rotation; each workgroup owns a slice of
@@ -631,7 +632,8 @@ int block_diag(scalit_ctx *c, int bjmax, double bjtol)
     for (int l = c->sF - 1; !c->scx && l >= 0; l--) {
         Level &L = c->lv[l];
         const bool layer = c->ndvr && l == c->sF - 1;
-        if (L.dim == 1 && !layer && jacobi_vec_fits(L.n)) {
+        const bool sym = !layer && L.h0_sym;
+        if (L.dim == 1 && sym && jacobi_vec_fits(L.n)) {
             SC_TRY(jacobi_level_vec(c, l, bjmax, bjtol, s));
         } else if (L.dim == 1 && sizeof(double) * (size_t)L.n * L.n > 160 * 1024) {
             SC_TRY(diag_level_dense(c, l, s));
@@ -642,7 +644,7 @@ int block_diag(scalit_ctx *c, int bjmax, double bjtol)
                                c->eig0.p, L.vosb.p, bjmax, bjtol, (int *)nullptr);
             HIP_TRY(hipGetLastError());
             HIP_TRY(hipStreamSynchronize(s));
-        } else if (!layer && jacobi_block_fits(L.n)) {
+        } else if (sym && jacobi_block_fits(L.n)) {
             SC_TRY(jacobi_level_block(c, l, bjmax, bjtol, s));
         } else {
             SC_TRY(diag_level_ndk<double>(c, l, bjmax, bjtol, layer ? c->outh.p : nullptr, L.h0.p,

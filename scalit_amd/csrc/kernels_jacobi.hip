@@ -34,8 +34,10 @@
 // at 64 x 96 x 80: 30 ms, against 679 ms with HOSB in memory and one launch
 // (level 3, 24.6 us each), one workgroup pass (level 2) or one wave's pass
 // (level 1) per rotation.  Those kernels (kernels_diag.hip) stay for what this
-// form does not hold: complex level matrices, the dense sNDVR layer, and
-// levels above 128 points (8-bit pair indices, 9 tiles of d for 16 waves).
+// form does not hold: complex level matrices, the dense sNDVR layer,
+// levels above 128 points (8-bit pair indices, 9 tiles of d for 16 waves), and an
+// H0 that is not symmetric (V(:,p) . U(:,q) would mix H0(p,q) and H0(q,p), of
+// which the reference reads one).
 #include "device_common.hpp"
 
 #include <algorithm>

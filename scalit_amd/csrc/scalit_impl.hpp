@@ -90,6 +90,7 @@ struct Level {
     DBuf<double> vosbt;
     DBuf<float> vosbt_f;
     bool has_h0 = false, has_dep = false;
+    bool h0_sym = false;   // H0 equals its transpose to rounding (scalit_set_h0)
     // complex level matrix and DEP (sCX = T), (re, im) adjacent: n x n
     // column-major and myDim values
     DBuf<double> h0cx, depcx;

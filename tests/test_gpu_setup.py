@@ -2,7 +2,8 @@
 of HosbDiag / MJACOBI at the sizes where its kernels change: tile edges and
 remainders, one-point levels, the R factor of the joint matrices (one chunk,
 several rounds, chunks in LDS and in memory), U in LDS or in memory, levels
-past the new kernels' sizes, levels with and without DEP, two to four levels.
+past the new kernels' sizes or not symmetric, levels with and without DEP, two to
+four levels.
 
 Tolerances (those of the other set-up tests): EIG0 1e-9, VOSB 1e-7, both
 relative to the largest entry.  The oracle's own sensitivity to a 1e-15
@@ -96,6 +97,22 @@ def test_setup_rotations_orthogonal(grid):
         d, ref = defect(v[l], n), defect(vo[l], n)
         print(grid, "level", l + 1, d, "oracle", ref, flush=True)
         assert d <= 1.25 * ref
+
+
+@pytest.mark.parametrize("sN,deps", [((7,), ()), ((12, 9), (1,)), ((6, 5, 4, 7), (1, 3)), ((10, 6, 40), (2,))])
+@pytest.mark.parametrize("asym", [0.05, 2e-17])
+def test_setup_nonsymmetric_levels(sN, deps, asym):
+    """Nonsymmetric level matrices, which the operator and its adjoint accept:
+    the set-up reads what MJACOBI reads of them (the upper triangle of a pair,
+    then columns mirrored into rows); and matrices symmetric but for rounding."""
+    g = P.rng(6)
+    h0, dep, dim = [], [], 1
+    for l, n in enumerate(sN):
+        a = g.standard_normal((n, n))
+        h0.append(0.05 * (a + a.T) + asym * g.standard_normal((n, n)) + np.diag(np.arange(n, dtype=float)))
+        dep.append(g.uniform(0.5, 1.5, size=dim) if l in deps else None)
+        dim *= n
+    _check(sN, h0, dep, g.standard_normal(dim))
 
 
 @pytest.mark.parametrize("bjmax,bjtol", [(0, 1e-5), (1, 1e-5), (3, 0.0), (1000, 1e-9)])
