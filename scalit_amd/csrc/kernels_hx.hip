@@ -725,8 +725,9 @@ struct VarA {
 };
 static const VarA kVarA[] = {{4, 1, 1}, {4, 3, 2}, {8, 3, 1}, {8, 2, 2}, {8, 1, 2}, {4, 2, 2}, {12, 2, 1}, {12, 1, 2}};
 constexpr int NVS = sizeof(kVarA) / sizeof(kVarA[0]);
-// two more, with the same results to the last bit: the pass tile by tile without
-// slabs in LDS (k_hx_levels12), and with mode 3 in it (k_hx_tile3, no pass B).
+// two more, with the same results to the last bit (BF16: the second rounds once less, see
+// variant_by_size): the pass tile by tile without slabs in LDS (k_hx_levels12), and with
+// mode 3 in it (k_hx_tile3, no pass B).
 // us of the whole operator with slabs / tiles / mode 3 in the tiles, FP64: 24x32x24, 1
 // vector 16.5 / 10.1 / 5.4 (the slab pass is bound by its staging); 37x50x41 30.7 /
 // 14.7 / 10.0; 64x96x80 28.4 / 22.0 / 37, 16 vectors 95 / 159 / -; 128x128x96 (T1 and
@@ -799,7 +800,8 @@ static void pass_a(scalit_ctx *c, int va, const T *t1, const T *t2, const T *res
 // the tile's points on the vector units, reading those points in every plane
 // (n3 times the reads of the mode-3 pass, from L2, instead of that pass's launch and
 // its read and write of Y).  The additions are in the order of the two passes
-// (bit for bit their results).  Bound by latency: TF3_J planes of a point and four
+// (bit for bit their results in FP64 and FP32; with BF16 storage Y is rounded once, by
+// the two passes also between them).  Bound by latency: TF3_J planes of a point and four
 // groups of each sum's operands are in flight.
 constexpr int TF3_J = 12;
 template <typename T, typename S>
@@ -950,6 +952,29 @@ static float time_calls(hipEvent_t e0, hipEvent_t e1, hipStream_t s, Fn fn)
     return hipGetLastError() == hipSuccess ? ms : 1e30f;
 }
 
+// The variant that the sizes decide, with nothing timed (a captured call cannot
+// time anything): the one-launch operator up to about one tile per SIMD.
+//
+// BF16 takes it by this rule only and never by a timing: it rounds Y once where the
+// two passes also round between them, so the choice shows in the result, which may not
+// depend on a timing or on a capture.  Its line is drawn where the two meet, us of the
+// whole operator, one launch / the faster pair: 28x36x28 8.6 / 10.6 for 7 vectors (1,176
+// tiles) and 12.1 / 11.2 for 9 (1,512), 20x20x20 8.0 / 10.8 for 14 (1,120) and 11.0 / 10.6 for
+// 24 (1,920), 100x20x16 9.8 / 10.9 for 5 (1,120) and 12.6 / 10.9 for 6 (1,344), 40x30x48 10.5 /
+// 10.7 for 4 (1,152), 32x32x56 10.1 / 10.8 for 4 (896) and 10.9 / 10.9 for 5 (1,120),
+// 24x32x64 10.5 / 10.7 for 2 (512) and 11.7 / 10.8 for 4 (1,024), 24x32x72 10.8 / 10.7 for one (288).
+template <typename T, typename S>
+static bool variant_by_size(const scalit_ctx *c, bool l2, int nvec, TuneEntry &e)
+{
+    if (!l2 || !tile3_fits<T>(c, nvec)) return false;
+    const long n1 = c->lv[0].n, n2 = c->lv[1].n, n3 = c->lv[2].n, cu = g_num_cu;
+    const long nt = ((n1 + 15) / 16) * ((n2 + 15) / 16) * n3 * nvec;
+    if (sizeof(S) < sizeof(T) ? !(n3 <= 64 && nt <= 5 * cu && nt * n3 <= 220 * cu) : !(n3 <= 48 && nt <= 4 * cu))
+        return false;
+    e.va = VA_FUSED;
+    return true;
+}
+
 template <typename T, typename S>
 static TuneEntry *tune(scalit_ctx *c, int prec, const T *t1, const T *t2, const T *l2, const T *dep, const T *res,
                        const T *sh, T sh0, int nvec, const S *x, long ldx, S *y, long ldy, hipStream_t s)
@@ -964,15 +989,13 @@ static TuneEntry *tune(scalit_ctx *c, int prec, const T *t1, const T *t2, const 
     const bool fuse = l2 && tile3_fits<T>(c, nvec);
     const int nva = fuse ? NVA : (tiles ? VA_FUSED : NVS);
     TuneEntry e{prec, nvec, fa >= 0 && fa < nva ? fa : 2, fb >= 0 && fb < (outer_tiles_fit((long)n1 * n2, n3, nvec, sizeof(T)) ? NVB : VB_TILES) ? fb : 0};
+    if (fa < 0 && fb < 0 && variant_by_size<T, S>(c, l2 != nullptr, nvec, e)) {
+        c->hx_tune.push_back(e);
+        return &c->hx_tune.back();
+    }
     if (st != hipStreamCaptureStatusNone) return nullptr;   // use the defaults, decide later
-    // up to one tile per SIMD the fused pass is faster than any pair of passes,
-    // so that nothing is timed (FP64, us: 24x32x24 with 4 vectors, 384 tiles, 6.4
-    // against 10.3 for the tile pass and pass B; 37x50x41 with 2 vectors, 984 tiles, 15.8
-    // against 18.1, with 4 vectors 24.0 against 21.9)
     const long nt = (long)((n1 + 15) / 16) * ((n2 + 15) / 16) * n3 * nvec;
-    if (fuse && fa < 0 && fb < 0 && nt <= 4L * g_num_cu && n3 <= 48) {
-        e.va = VA_FUSED;
-    } else if (fa < 0 || fb < 0) {
+    if (fa < 0 || fb < 0) {
         hipEvent_t e0, e1;
         if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) return nullptr;
         float best = 1e30f, best_b = 1e30f;
@@ -996,7 +1019,7 @@ static TuneEntry *tune(scalit_ctx *c, int prec, const T *t1, const T *t2, const 
                 e.vb = vb;
             }
         }
-        if (fuse && fa < 0 && fb < 0 && nt <= 8L * g_num_cu &&   // past that it is far behind
+        if (fuse && sizeof(S) == sizeof(T) && fa < 0 && fb < 0 && nt <= 8L * g_num_cu &&   // past that it is far behind
             time_calls(e0, e1, s, [&] {
                 pass_fused<T, S>(c, t1, t2, l2, dep, res, sh, sh0, nvec, x, ldx, y, ldy, nullptr, s);
             }) < best + best_b)

@@ -137,6 +137,70 @@ def test_three_levels_by_tiles(monkeypatch, sN, nvec, va, vb):
     ctx.close()
 
 
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("sN,nvec", [((5, 3, 2), 1), ((16, 16, 1), 2), ((17, 33, 7), 3), ((24, 32, 24), 1),
+                                     ((20, 18, 50), 16), ((37, 50, 41), 2), ((7, 9, 128), 3)])
+def test_three_level_variants_agree(monkeypatch, sN, nvec, dt):
+    """Every variant of the 3-level operator that a timing picks from gives the
+    same bits for every stored type: the default slab pass with each form of
+    pass B, another slab shape, the tile pass with each form, and, in FP64 and
+    FP32, mode 3 in the tiles."""
+    prob = P.build_problem(*sN, P.gaussian_potential(5), seed=5)
+    ref = None
+    for va, vb in ((2, 0), (2, 1), (2, 2), (2, 3), (7, 0), (8, 0), (8, 3), (9, 0)):
+        if va == 9 and dt == torch.bfloat16:
+            continue
+        monkeypatch.setenv("SCALIT_HX_VARIANT_A", str(va))
+        monkeypatch.setenv("SCALIT_HX_VARIANT_B", str(vb))
+        ctx = Context.from_problem(prob, e0=0.01)
+        x = ctx.to_device(P.random_vectors(ctx.N, nvec, 9), dt)
+        y = ctx.hx(x, L.TA1) if dt == torch.float64 else ctx.hx_lp(x, L.TA1)
+        assert ctx.hx_variant({torch.float64: L.FP64, torch.float32: L.FP32, torch.bfloat16: L.BF16}[dt], nvec) == (va, vb)
+        ref = y if ref is None else ref
+        assert torch.equal(y, ref), (va, vb, int((y != ref).sum()))
+        ctx.close()
+
+
+@pytest.mark.parametrize("sN,nvec,fused", [((24, 32, 24), 1, True), ((12, 14, 10), 120, True), ((32, 32, 56), 4, True),
+                                           ((12, 14, 10), 150, False), ((20, 20, 20), 17, False),
+                                           ((32, 32, 64), 4, False), ((16, 20, 70), 1, False)])
+def test_bf16_variant_by_size(monkeypatch, sN, nvec, fused):
+    """BF16 storage: the one-launch operator rounds Y once and the two passes
+    twice, so that the sizes and not a timing decide: on either side of the line
+    the default call gives the bits of that form."""
+    prob = P.build_problem(*sN, P.gaussian_potential(5), seed=5)
+    ys = []
+    for va in (None, 9 if fused else 2):
+        if va is not None:
+            monkeypatch.setenv("SCALIT_HX_VARIANT_A", str(va))
+            monkeypatch.setenv("SCALIT_HX_VARIANT_B", "0")
+        ctx = Context.from_problem(prob, e0=0.01)
+        ys.append(ctx.hx_lp(ctx.to_device(P.random_vectors(ctx.N, nvec, 9), torch.bfloat16), L.TA1))
+        ctx.close()
+    assert torch.equal(*ys)
+
+
+@pytest.mark.parametrize("sN,nvec", [((24, 32, 24), 1), ((37, 50, 41), 2), ((20, 20, 20), 17), ((16, 20, 70), 1)])
+def test_captured_call_agrees(sN, nvec):
+    """A recorded call of a batch size that was never applied before, which times
+    nothing, and an eager call, which may, give the same bits on every replay."""
+    prob = P.build_problem(*sN, P.gaussian_potential(5), seed=5)
+    ctx, eager = Context.from_problem(prob, e0=0.01), Context.from_problem(prob, e0=0.01)
+    x = ctx.to_device(P.random_vectors(ctx.N, nvec, 9))
+    y = torch.empty_like(x)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        ctx.hx(x, L.TA1, out=y)
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(eager.hx(x, L.TA1), y)
+    ctx.close()
+    eager.close()
+
+
 @pytest.mark.parametrize("sN,nvec", [((5, 3, 2), 1), ((16, 17, 16), 2), ((24, 32, 24), 3), ((7, 130, 3), 2),
                                      ((70, 40, 9), 1)])
 def test_rotations_by_tiles(sN, nvec):
