@@ -953,7 +953,18 @@ static float time_calls(hipEvent_t e0, hipEvent_t e1, hipStream_t s, Fn fn)
 }
 
 // The variant that the sizes decide, with nothing timed (a captured call cannot
-// time anything): the one-launch operator up to about one tile per SIMD.
+// time anything): up to about one tile per SIMD the one-launch operator, or the
+// tile forms of both passes where it has more to read (it reads every point
+// of a tile in n3 planes).
+//
+// FP64, us of the whole operator, one launch / the faster pair (tiles x n3):
+// 28x36x28 8.9 / 10.3 for 4 vectors (19 k), 11.4 / 11.7 for 5 (24 k), 12.2 / 11.7 for 6 (28 k);
+// 48x64x40 9.2 / 10.3 for one (19 k), 14.9 / 14.1 for two (38 k); 37x50x41 9.5 / 10.2 (20 k),
+// 15.2 / 12.7 (40 k); 17x23x47 9.6 / 10.6 for 3 (27 k), 10.6 / 10.4 for 4 (35 k), 15.4 / 10.4 for 5
+// (44 k); 40x30x48 10.8 / 10.4 for two (28 k), 15.6 / 11.7 for 3 (41 k).  The faster pair is the
+// tile forms in all of these.  FP32: the one launch up to 4 tiles per CU (48x64x40 with two
+// vectors 9.0 / 10.8, 40x30x48 with 3 10.1 / 10.7).  From 49 planes on the two are timed
+// (24x32x64 with two vectors 11.1 / 10.3 in FP64 and 9.7 / 10.8 in FP32).
 //
 // BF16 takes it by this rule only and never by a timing: it rounds Y once where the
 // two passes also round between them, so the choice shows in the result, which may not
@@ -972,6 +983,10 @@ static bool variant_by_size(const scalit_ctx *c, bool l2, int nvec, TuneEntry &e
     if (sizeof(S) < sizeof(T) ? !(n3 <= 64 && nt <= 5 * cu && nt * n3 <= 220 * cu) : !(n3 <= 48 && nt <= 4 * cu))
         return false;
     e.va = VA_FUSED;
+    if (sizeof(T) == 8 && nt * n3 > 112 * cu && outer_tiles_fit(n1 * n2, n3, nvec, sizeof(T))) {
+        e.va = VA_TILES;
+        e.vb = VB_TILES;
+    }
     return true;
 }
 

@@ -180,6 +180,25 @@ def test_bf16_variant_by_size(monkeypatch, sN, nvec, fused):
     assert torch.equal(*ys)
 
 
+@pytest.mark.parametrize("sN,nvec,variant", [((24, 32, 24), 1, (9, 0)), ((28, 36, 28), 6, (9, 0)),
+                                             ((48, 64, 40), 2, (8, 3)), ((17, 23, 47), 5, (8, 3))])
+def test_fp64_variant_by_size(monkeypatch, sN, nvec, variant):
+    """The one-launch operator and, on the other side of its line, the tile forms
+    of both passes: the slab pass's bits."""
+    prob = P.build_problem(*sN, P.gaussian_potential(5), seed=5)
+    ys = []
+    for va in (None, 2):
+        if va is not None:
+            monkeypatch.setenv("SCALIT_HX_VARIANT_A", str(va))
+            monkeypatch.setenv("SCALIT_HX_VARIANT_B", "0")
+        ctx = Context.from_problem(prob, e0=0.01)
+        ys.append(ctx.hx(ctx.to_device(P.random_vectors(ctx.N, nvec, 9)), L.TA1))
+        if va is None:
+            assert ctx.hx_variant(L.FP64, nvec) == variant
+        ctx.close()
+    assert torch.equal(*ys)
+
+
 @pytest.mark.parametrize("sN,nvec", [((24, 32, 24), 1), ((37, 50, 41), 2), ((20, 20, 20), 17), ((16, 20, 70), 1)])
 def test_captured_call_agrees(sN, nvec):
     """A recorded call of a batch size that was never applied before, which times
