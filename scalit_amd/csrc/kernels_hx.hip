@@ -723,8 +723,9 @@ bool fast3_supported(const scalit_ctx *c)
 struct VarA {
     int waves, rb, cb;
 };
-static const VarA kVarA[] = {{4, 1, 1}, {4, 3, 2}, {8, 3, 1}, {8, 2, 2}, {8, 1, 2}, {4, 2, 2}, {12, 2, 1}, {12, 1, 2}};
+static const VarA kVarA[] = {{4, 1, 1}, {8, 3, 1}, {8, 2, 2}, {8, 1, 2}, {12, 2, 1}, {12, 1, 2}};
 constexpr int NVS = sizeof(kVarA) / sizeof(kVarA[0]);
+constexpr int VA_DEF = 1;   // before anything is timed
 // two more, with the same results to the last bit (BF16: the second rounds once less, see
 // variant_by_size): the pass tile by tile without slabs in LDS (k_hx_levels12), and with
 // mode 3 in it (k_hx_tile3, no pass B).
@@ -758,12 +759,10 @@ static void launch_a(int va, dim3 g, size_t lds, hipStream_t s, int n1, int n2, 
     launch_a1<T, S, TL, W, RB, CB>(g, lds, s, n1, n2, n3, nvec, t1, t2, res, sh, sh0, x, ldx, y, ldy, act)
     switch (va) {
     case 0: LA(4, 1, 1); break;
-    case 1: LA(4, 3, 2); break;
-    case 2: LA(8, 3, 1); break;
-    case 3: LA(8, 2, 2); break;
-    case 4: LA(8, 1, 2); break;
-    case 5: LA(4, 2, 2); break;
-    case 6: LA(12, 2, 1); break;
+    case 1: LA(8, 3, 1); break;
+    case 2: LA(8, 2, 2); break;
+    case 3: LA(8, 1, 2); break;
+    case 4: LA(12, 2, 1); break;
     default: LA(12, 1, 2); break;
     }
 #undef LA
@@ -1003,7 +1002,7 @@ static TuneEntry *tune(scalit_ctx *c, int prec, const T *t1, const T *t2, const 
     const bool tiles = levels12_fits(n1, n2, n3, nvec, sizeof(T));
     const bool fuse = l2 && tile3_fits<T>(c, nvec);
     const int nva = fuse ? NVA : (tiles ? VA_FUSED : NVS);
-    TuneEntry e{prec, nvec, fa >= 0 && fa < nva ? fa : 2, fb >= 0 && fb < (outer_tiles_fit((long)n1 * n2, n3, nvec, sizeof(T)) ? NVB : VB_TILES) ? fb : 0};
+    TuneEntry e{prec, nvec, fa >= 0 && fa < nva ? fa : VA_DEF, fb >= 0 && fb < (outer_tiles_fit((long)n1 * n2, n3, nvec, sizeof(T)) ? NVB : VB_TILES) ? fb : 0};
     if (fa < 0 && fb < 0 && variant_by_size<T, S>(c, l2 != nullptr, nvec, e)) {
         c->hx_tune.push_back(e);
         return &c->hx_tune.back();
@@ -1015,7 +1014,6 @@ static TuneEntry *tune(scalit_ctx *c, int prec, const T *t1, const T *t2, const 
         if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) return nullptr;
         float best = 1e30f, best_b = 1e30f;
         for (int va = 0; va < std::min(nva, VA_FUSED) && fa < 0; va++) {
-            if (va == 1 || va == 5) continue;   // 4 waves of 3x2 or 2x2 tiles: never the fastest at any size tried
             const float ms = time_calls(e0, e1, s, [&] {
                 pass_a<T, S>(c, va, t1, t2, res, sh, sh0, nvec, x, ldx, y, ldy, nullptr, s);
             });
@@ -1055,7 +1053,7 @@ static int hx_fast3(scalit_ctx *c, int prec, const T *t1, const T *t2, const T *
 {
     const int n1 = c->lv[0].n, n2 = c->lv[1].n, n3 = c->lv[2].n;
     TuneEntry *te = tune<T, S>(c, prec, t1, t2, l2, dep, res, shifts, shift0, nvec, x, ldx, y, ldy, s);
-    const int va = te ? te->va : 2, vb = te ? te->vb : 0;
+    const int va = te ? te->va : VA_DEF, vb = te ? te->vb : 0;
     if (va == VA_FUSED && l2) {
         pass_fused<T, S>(c, t1, t2, l2, dep, res, shifts, shift0, nvec, x, ldx, y, ldy, active, s);
         HIP_TRY(hipGetLastError());
@@ -1226,7 +1224,7 @@ int hx_pass_f64(scalit_ctx *c, int pass, int nvec, const double *x, long ldx, do
     const int n1 = L[0].n, n2 = L[1].n, n3 = L[2].n;
     TuneEntry *te = tune<double, double>(c, SCALIT_FP64, L[0].h0.p, L[1].h0.p, L[2].h0.p, L[2].depv.p, c->res.p,
                                          nullptr, 0.0, nvec, x, ldx, y, ldy, s);
-    const int va = te ? te->va : 2, vb = te ? te->vb : 0;
+    const int va = te ? te->va : VA_DEF, vb = te ? te->vb : 0;
     if (pass == 1)
         pass_a<double, double>(c, va, L[0].h0.p, L[1].h0.p, c->res.p, nullptr, 0.0, nvec, x, ldx, y, ldy, nullptr, s);
     else if (pass == 2)

@@ -293,17 +293,18 @@ def test_px_large_level1_blocks(grid, nv):
 
 def test_hx_bench_shape_every_variant(monkeypatch):
     """The bench workload's exact shape, 64 x 96 x 80 at batch 16, through
-    every pass-A block shape and pass-B width the autotuner can pick (forced
-    one pair at a time), FP64 within 1e-12 and FP32 within 2e-6 of the oracle
-    on the first, a middle and the last vector of the batch."""
+    every pass-A block shape, the tile pass and every form of pass B that the
+    autotuner times there (forced one pair at a time), FP64 within 1e-12 and
+    FP32 within 2e-6 of the oracle on the first, a middle and the last vector of
+    the batch."""
     grid, nv = (64, 96, 80), 16
     prob = P.build_problem(*grid, P.gaussian_potential(5), seed=5)
     op = O.Operator(prob.sN, prob.h0, prob.res, prob.dep)
     x = P.random_vectors(prob.N, nv, 21)
     check = (0, 7, 15)
     ref = {b: op.hx(x[b]) for b in check}
-    for va in range(8):
-        for vb in range(3):
+    for va in range(7):
+        for vb in range(4):
             print(f"hx variant A={va} B={vb}", flush=True)
             monkeypatch.setenv("SCALIT_HX_VARIANT_A", str(va))
             monkeypatch.setenv("SCALIT_HX_VARIANT_B", str(vb))
