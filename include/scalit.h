@@ -391,8 +391,8 @@ int scalit_debug_sym_eig(int n, const double *a, int lda, double *w, double *z, 
  * ns[j] x ns[j] block of a + j lda lda (host, column-major, leading dimension
  * lda, upper triangle read); its eigenvalues, ascending, go to w + j lda. */
 int scalit_debug_sym_eigvals_batch(int njobs, const int *ns, const double *a, int lda, double *w);
-/* The fused H*X kernel variants (pass A block shape, pass B width) the
- * autotuner picked for this precision and batch size (tuning them if needed). */
+/* The fused H*X kernel variants (form of pass A, form of pass B) the sizes or
+ * the autotuner picked for this precision and batch size (tuning them if needed). */
 int scalit_debug_hx_variant(scalit_ctx *ctx, int prec, int nvec, int *va, int *vb);
 /* Launch one pass of the fused FP64 H*X alone (1: modes 1+2 and the diagonal,
  * 2: mode 3 accumulate) so that each kernel can be timed by itself. */

@@ -226,6 +226,20 @@ def test_rotations_by_tiles(sN, nvec):
     """P*X with the level >= 2 rotations tile by tile (also past 128 points), on
     seeded orthogonal rotations, against dense products; FP64 1e-12, FP32 1e-5
     (the shift lies below every EIG0, so the divide amplifies nothing)."""
+    _check_px(sN, [nvec])
+
+
+# each row: the sizes of one register form of the level-1 kernel's prefetch, with MFMA
+# (8 vectors and more, or more than 256 outputs) and on the vector units
+@pytest.mark.parametrize("n1", [20, 64, 65, 80, 81, 96, 97, 111, 112, 113, 128])
+def test_px_level1_forms(n1):
+    """P*X at the edges of level 1's forms: the largest block of a prefetch and
+    one more, past the prefetch (113, 128), and batches on both sides of the MFMA
+    rule, with a shift per vector; tolerances as above."""
+    _check_px((n1, 3, 2), [1, 2, 3, 4, 5, 7, 8, 17])
+
+
+def _check_px(sN, batches):
     g = P.rng(4)
     ctx = Context(sN, [False] * len(sN))
     n = ctx.N
@@ -237,19 +251,22 @@ def test_rotations_by_tiles(sN, nvec):
     ctx.set_precond(vosb, eig0)
     ctx.set_res(np.zeros(n))
     ctx.set_shift(0.5)
-    x = P.random_vectors(n, nvec, 12)
 
     def rot(z, l, trans):
         q = vosb[l].reshape(ctx.blk[l], sN[l], sN[l]).transpose(0, 2, 1)
-        z = z.reshape(nvec, ctx.blk[l], sN[l], ctx.dim[l])
-        return np.einsum("bji,vbjk->vbik" if trans else "bij,vbjk->vbik", q, z).reshape(nvec, n)
+        z = z.reshape(-1, ctx.blk[l], sN[l], ctx.dim[l])
+        return np.einsum("bji,vbjk->vbik" if trans else "bij,vbjk->vbik", q, z).reshape(-1, n)
 
-    z = x
-    for l in (2, 1, 0):
-        z = rot(z, l, True)
-    z = z / (eig0 - 0.5)
-    for l in (0, 1, 2):
-        z = rot(z, l, False)
-    assert _rel(ctx.px(ctx.to_device(x)).cpu().numpy(), z) <= 1e-12
-    assert _rel(ctx.px_lp(ctx.to_device(x, torch.float32)).double().cpu().numpy(), z) <= 1e-5
+    for nvec in batches:
+        x = P.random_vectors(n, nvec, 12)
+        for sh in (None, np.linspace(-0.5, 0.5, nvec)):
+            z = x
+            for l in reversed(range(len(sN))):
+                z = rot(z, l, True)
+            z = z / (eig0 - (0.5 if sh is None else sh[:, None]))
+            for l in range(len(sN)):
+                z = rot(z, l, False)
+            assert _rel(ctx.px(ctx.to_device(x), shifts=sh).cpu().numpy(), z) <= 1e-12, (nvec, sh)
+            y = ctx.px_lp(ctx.to_device(x, torch.float32), shifts=sh)
+            assert _rel(y.double().cpu().numpy(), z) <= 1e-5, (nvec, sh)
     ctx.close()

@@ -269,9 +269,10 @@ def _precond_from_gpu(ctx, op):
 
 @pytest.mark.parametrize("grid,nv", [((80, 96, 64), 1), ((80, 96, 64), 16), ((128, 128, 96), 1)])
 def test_px_large_level1_blocks(grid, nv):
-    """Level-1 rotations larger than 64: the BIG forms of k_px_l1, on the MFMA
-    path for n1 = 80 at batch 16 and on the VALU path for n1 = 80 at batch 1
-    and n1 = 128, TOSB and TOSBD2, FP64 (1e-12) and FP32 (1e-4)."""
+    """Level-1 rotations larger than 64: the whole-block prefetch of k_px_l1 for
+    n1 = 80, on MFMA at batch 16 and on the vector units at batch 1, and n1 = 128,
+    whose last values load while a block is staged, TOSB and TOSBD2, FP64 (1e-12)
+    and FP32 (1e-4)."""
     print(f"px large blocks grid={grid} nv={nv}", flush=True)
     prob, op, ctx = setup(grid, e0=-0.02)
     _precond_from_gpu(ctx, op)

@@ -37,9 +37,9 @@ def _check(sN, h0, dep, res, bjmax=1000, bjtol=1e-5):
     print(sN, "VOSB", errs, "EIG0", ee, flush=True)
     assert ee <= 1e-9
     assert max(errs) <= 1e-7
-    for l, n in enumerate(sN):   # the last block's rotation stays orthogonal
-        w = v[l][-n * n:].reshape(n, n, order="F")
-        assert np.abs(w.T @ w - np.eye(n)).max() <= 1e-12
+    for l, n in enumerate(sN):   # every block's rotation stays orthogonal
+        w = np.asarray(v[l]).reshape(-1, n, n)   # rows: the columns of V
+        assert np.abs(w @ w.transpose(0, 2, 1) - np.eye(n)).max() <= 1e-12
     ctx.close()
 
 
@@ -50,9 +50,18 @@ def _check(sN, h0, dep, res, bjmax=1000, bjtol=1e-5):
     (33, 31, 7),      # odd sizes below and above a tile
     (48, 16, 40),     # level 3: R factor in two rounds, chunks in LDS
     (40, 65, 4),      # five tiles along level 2, fewer points than its size
+    (4, 81, 3),       # six tiles along level 2, one point into the sixth
+    (4, 96, 5),       # six full tiles
+    (12, 9, 80),      # five tiles and the R factor along level 3
+    (12, 9, 96),      # six
     (3, 100, 9),      # U in memory
     (20, 9, 97),      # R factor (180 > 98) with U in memory
     (30, 20, 110),    # R factor in two rounds, chunks in memory
+    (65, 3, 2),       # level 1: rows of 5 values a lane, of 6 (81, 96) and of 8 (100)
+    (80, 3, 2),
+    (81, 3, 2),
+    (96, 2, 2),
+    (100, 2, 2),      # the largest with V in LDS
     (101, 3, 2),      # level 1 with V in memory
     (128, 2, 2),      # its largest size
     (140, 2, 2),      # level 1 past it: one wave per block
