@@ -150,7 +150,9 @@ int scalit_get_precond(scalit_ctx *ctx, double *const *vosb, double *eig0);
 int scalit_hx(scalit_ctx *ctx, int ntype, int nvec, const double *x, long ldx, double *y, long ldy,
               const double *shifts, scalit_stream stream);
 /* The same product in fp32 (prec SCALIT_FP32: float vectors) or with bf16
- * storage (SCALIT_BF16: unsigned short vectors), fp32 accumulation. */
+ * storage (SCALIT_BF16: unsigned short vectors), fp32 accumulation.  BF16: a
+ * small operator and batch round Y once, larger ones also once before the last
+ * level is added; the sizes decide which. */
 int scalit_hx_lp(scalit_ctx *ctx, int prec, int ntype, int nvec, const void *x, long ldx, void *y, long ldy,
                  const float *shifts, scalit_stream stream);
 /* Adjoint of H*X for gradients: dx_b = H^T g_b (H0 transposed per level; RES

@@ -19,9 +19,9 @@ LIB = os.path.join(HERE, "libscalit_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-SOURCES = ["kernels_hx.hip", "kernels_px.hip", "kernels_diag.hip", "kernels_jacobi.hip", "kernels_vec.hip", "solvers.hip", "capi.hip",
-           "noalloc.hip", "truncate.hip", "kernels_qmr.hip", "osbw.hip", "complex.hip", "complex_h0.hip",
-           "formats.cpp"]
+SOURCES = ["kernels_hx.hip", "kernels_px.hip", "kernels_diag.hip", "kernels_jacobi.hip", "kernels_vec.hip",
+           "solvers.hip", "capi.hip", "noalloc.hip", "truncate.hip", "kernels_qmr.hip", "osbw.hip", "complex.hip",
+           "complex_h0.hip", "formats.cpp"]
 
 FLAGS = [
     f"--offload-arch={ARCH}",

@@ -16,10 +16,11 @@
 // Vectors are split (N real parts, then N imaginary parts, per vector); the
 // level matrices keep the reference's (re, im) pairs.  The products run on FP64
 // MFMA: the diagonal and levels 1 and 2 in one pass, each further level in one
-// that adds to Y.  MYHX_CX of one vector at 64 x 96 x 80: 29 us (levels 1 and 2: 19, level 3: 13), against 121 us
-// with one thread per output point (k_cxh_level_lds: 40 us per level, bound by a
-// load of H0CX per multiply-add), which stays for a level of one column
-// per block (one-level operators, and level 1 under a dense sNDVR layer).
+// that adds to Y.  MYHX_CX of one vector at 64 x 96 x 80, passes back to back: 29 us (each
+// by itself under the profiler: levels 1 and 2 19.0 with the matrix pipe 31% busy, level 3 12.8
+// with 20%), against 121 us with one thread per output point (k_cxh_level_lds: 40 us
+// per level, bound by a load of H0CX per multiply-add), which stays for a level of one
+// column per block (one-level operators, and level 1 under a dense sNDVR layer).
 #include "device_common.hpp"
 #include "solver_state.hpp"
 

@@ -387,7 +387,8 @@ static int hx_generic(scalit_ctx *c, const T *res, const T *shifts, T shift0, in
     int l = 0;
     const Level *L = c->lv;
     if (c->sF >= 2 + (c->ndvr ? 1 : 0) && levels12_fits(L[0].n, L[1].n, L[1].blk, nvec, sizeof(T))) {
-        launch_levels12<T, S, false>(L[0].n, L[1].n, L[1].blk, nvec, h[0], h[1], dep[1], res, shifts, shift0, x, ldx, y, ldy, active, s);
+        launch_levels12<T, S, false>(L[0].n, L[1].n, L[1].blk, nvec, h[0], h[1], dep[1], res, shifts, shift0, x, ldx,
+                                     y, ldy, active, s);
         l = 2;
     } else {
         hipLaunchKernelGGL((k_diag_init<T, S>), g, dim3(th), 0, s, c->N, res, shifts, shift0, x, ldx, y, ldy, active);
@@ -731,7 +732,7 @@ constexpr int VA_DEF = 1;   // before anything is timed
 // mode 3 in it (k_hx_tile3, no pass B).
 // us of the whole operator with slabs / tiles / mode 3 in the tiles, FP64: 24x32x24, 1
 // vector 16.5 / 10.1 / 5.4 (the slab pass is bound by its staging); 37x50x41 30.7 /
-// 14.7 / 10.0; 64x96x80 28.4 / 22.0 / 37, 16 vectors 95 / 159 / -; 128x128x96 (T1 and
+// 10.2 / 9.5; 64x96x80 28.4 / 22.0 / 37, 16 vectors 95 / 159 / -; 128x128x96 (T1 and
 // T2 do not fit beside the slab) 84 / 52 / -, 4 vectors in FP32 106 / 73 / -.
 constexpr int VA_TILES = NVS, VA_FUSED = NVS + 1;
 constexpr int NVA = NVS + 2;
@@ -1002,7 +1003,8 @@ static TuneEntry *tune(scalit_ctx *c, int prec, const T *t1, const T *t2, const 
     const bool tiles = levels12_fits(n1, n2, n3, nvec, sizeof(T));
     const bool fuse = l2 && tile3_fits<T>(c, nvec);
     const int nva = fuse ? NVA : (tiles ? VA_FUSED : NVS);
-    TuneEntry e{prec, nvec, fa >= 0 && fa < nva ? fa : VA_DEF, fb >= 0 && fb < (outer_tiles_fit((long)n1 * n2, n3, nvec, sizeof(T)) ? NVB : VB_TILES) ? fb : 0};
+    const int nvb = outer_tiles_fit((long)n1 * n2, n3, nvec, sizeof(T)) ? NVB : VB_TILES;
+    TuneEntry e{prec, nvec, fa >= 0 && fa < nva ? fa : VA_DEF, fb >= 0 && fb < nvb ? fb : 0};
     if (fa < 0 && fb < 0 && variant_by_size<T, S>(c, l2 != nullptr, nvec, e)) {
         c->hx_tune.push_back(e);
         return &c->hx_tune.back();
@@ -1022,8 +1024,7 @@ static TuneEntry *tune(scalit_ctx *c, int prec, const T *t1, const T *t2, const 
                 e.va = va;
             }
         }
-        for (int vb = 0; vb < NVB && fb < 0 && l2; vb++) {
-            if (vb == VB_TILES && !outer_tiles_fit((long)n1 * n2, n3, nvec, sizeof(T))) continue;
+        for (int vb = 0; vb < nvb && fb < 0 && l2; vb++) {
             const float ms = time_calls(e0, e1, s, [&] {
                 launch_b<T, S>(vb, n1, n2, n3, nvec, l2, dep, x, ldx, y, ldy, nullptr, s);
             });

@@ -30,10 +30,11 @@
 //    squares after the rotation, from the A, B, C of the angle.
 //
 // What bounds it: the serial chain of steps (a few hundred per sweep, each a
-// handful of dependent LDS, MFMA and square-root latencies).  The whole set-up
-// at 64 x 96 x 80: 30 ms, against 679 ms with HOSB in memory and one launch
-// (level 3, 24.6 us each), one workgroup pass (level 2) or one wave's pass
-// (level 1) per rotation.  Those kernels (kernels_diag.hip) stay for what this
+// handful of dependent LDS, MFMA and square-root latencies; the matrix pipe is 6% busy in
+// level 2 at 64 x 96 x 80).  The set-up there: level 1 11.7 ms, level 2 6.4, level 3 4.2 and
+// 1.1 for its R factor; 25 to 29 ms with the first P*X, against 679 with HOSB in memory
+// and one launch (level 3, 24.6 us each), one workgroup pass (level 2) or one wave's
+// pass (level 1) per rotation.  Those kernels (kernels_diag.hip) stay for what this
 // form does not hold: complex level matrices, the dense sNDVR layer,
 // levels above 128 points (8-bit pair indices, 9 tiles of d for 16 waves), and an
 // H0 that is not symmetric (V(:,p) . U(:,q) would mix H0(p,q) and H0(q,p), of
@@ -58,7 +59,7 @@ struct Rot {
 // third-order and a second-order step, and s corrected by its own residual (a few
 // dependent operations each where the library's square root and division take
 // several times as many; the rotations of a step wait for them: level 1 at
-// 64 x 96 x 80 13.7 -> 11.5 ms)
+// 64 x 96 x 80 13.7 -> 11.7 ms)
 __device__ __forceinline__ void rsqrt_unit(double x, double &r, double &s)
 {
     double y = __builtin_amdgcn_rsq(x);
@@ -625,6 +626,8 @@ int jacobi_level_vec(scalit_ctx *c, int l, int bjmax, double bjtol, hipStream_t 
     DBuf<int> cnt;
     DBuf<unsigned short> pairs;
     SC_TRY(upload_schedule(sc, cnt, pairs, s));
+    // values per lane: the next built count (3 and 7 are not built: 33 to 48 points run
+    // as 64, 97 to 112 as 128)
 #define JV(KL) launch_vec<KL>(L.n, L.blk, sc, pairs.p, L.h0.p, c->eig0.p, L.vosb.p, bjmax, bjtol, s)
     const int kl = (L.n + 15) / 16;
     if (kl <= 2) JV(2);
@@ -724,6 +727,7 @@ int jacobi_level_block(scalit_ctx *c, int l, int bjmax, double bjtol, hipStream_
         bse = bsd = (long)nc * nc;
     }
     SC_TRY(dg.alloc((size_t)((nd + 15) / 16 * 16) * n * nblk));
+    // tiles along n: the next built count (3 and 7 are not built here either)
 #define JB(NR)                                                                                                      \
     launch_block<NR>(n, nd, nblk, sc, cnt.p, pairs.p, L.h0.p, E, lde, bse, dd, bsd, dg.p, ug, L.vosb.p, wii.p, bjmax, \
                      bjtol, s)

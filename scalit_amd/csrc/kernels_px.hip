@@ -16,7 +16,8 @@
 // whole iteration.  V1^T, the divide and V1 are adjacent in the sequence, so
 // one kernel applies all three per block and VOSB level 1 is read once per
 // P*X for all vectors of a batch: on MFMA with the vectors as the 16 columns
-// of a tile (batches of 8 and more), or one wave per vector on the VALU.
+// of a tile (batches of 8 and more, and more outputs per block than threads), or on
+// the VALU with a thread or several per output.
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -76,9 +77,11 @@ __global__ void k_rotate_generic(int nin, int nout, int blk, const T *__restrict
 // the shifts and activity of the first chunk of vectors and of the current
 // later one (2 WC each).  NP: the block size the registers of the prefetch hold (64,
 // 80, 96 or 112: (NP / 16)^2 rotation values and NP / 16 first-chunk values per thread); with
-// larger blocks (n1 > 112, VALU) the rest is loaded while it is staged.  Prefetching
-// a whole block of 80 points instead of its first 4,096 values took this kernel from 90 to 79 us at 80x96x64 with 16
-// FP32 vectors, and the whole P*X of one FP64 vector there from 153 to 112 us.
+// larger blocks (n1 > 112, VALU) the rest is loaded while it is staged.
+// Prefetching a whole block of 80 points instead of its first 4,096 values took this
+// kernel from 90 to 79 us at 80x96x64 with 16 FP32 vectors (19 vector instructions per
+// MFMA, the matrix pipe 21% busy), and the whole P*X of one FP64 vector there from 153
+// to 112 us.
 template <typename T, typename S, typename SO, bool MF, int NP>
 __global__ void __launch_bounds__(256) k_px_l1(int n1, int nblk, int nvec, const T *__restrict__ vosb,
                                                const T *__restrict__ eig0, const T *__restrict__ shifts, T shift0,

@@ -942,9 +942,16 @@ __global__ void __launch_bounds__(QP_NT) k_pist_persist(PpArgs pa)
 // Whether the persistent solvers take this operator: the fused 3-level
 // layout (sF = 3, DEP on level 3 only, no sNDVR layer) with its
 // preconditioner, levels of at most QP_NMAX points, at most 65,536 points and
-// theta planes of at most 1,536 points.  Past that a plane's phase is longer than
-// the launches it saves (measured: 81 against 113 us per QMR iteration at
-// 32x40x24, 151 against 121 at 40x48x32).
+// theta planes of at most 1,536 points.  A plane's phase grows with n1^2 n2 and
+// with the right-hand sides, and the line is drawn for what a job runs most, the
+// PIST of one window, persistent / one launch per step, ms for the lowest 20
+// levels: 16x20x12 21.7 / 36.3, 24x32x24 44 / 80, 32x40x24 65 / 92, 32x48x32 82 / 98, 40x36x24
+// 76 / 95, 48x28x30 72 / 86; past it 40x48x32 119 / 106, and inside it 48x32x40 121 / 106.
+// Several right-hand sides meet earlier: PIST of 4 windows 24x32x24 6.4 / 7.7, 28x36x28
+// 8.0 / 8.9, 32x40x24 9.2 / 8.8, of 12 windows 16x20x12 9.1 / 8.5, 24x32x24 19 / 14.  So do
+// solves without Krylov steps around them, us per QMR iteration: one right-hand
+// side 24x32x24 50 / 68, 32x32x24 64 / 68, 32x40x24 80 / 70, 48x32x40 153 / 85; four 24x32x24
+// 72 / 73, 32x40x24 105 / 82.
 bool qmr_persist_ok(const scalit_ctx *c)
 {
     if (!c->fast3 || c->ndvr || c->sF != 3 || !c->has_precond || !c->has_res) return false;

@@ -7,9 +7,10 @@
 //
 // Persistent grid (x: workgroups per block, y: block): each workgroup stages
 // its block's A in LDS once; each wave then walks its own tiles of 16
-// consecutive p of one vector (no workgroup barrier after the staging) and loads the next tile's X and d into registers while the
-// current tile's MFMAs run (Y, when adding, at the top of its own tile).  Lane (lr, lk) of a tile holds X(p0 + lr, 4 s + lk)
-// for all s (the B fragments); the A fragments come from LDS.  NR = tiles of
+// consecutive p of one vector (no workgroup barrier after the staging) and
+// loads the next tile's X and d into registers while the current tile's MFMAs
+// run (Y, when adding, at the top of its own tile).  Lane (lr, lk) of a tile
+// holds X(p0 + lr, 4 s + lk) for all s (the B fragments); the A fragments come from LDS.  NR = tiles of
 // 16 along n (n <= 16 NR, A zero padded), a compile-time count so the register
 // arrays hold exactly one column.
 #pragma once
