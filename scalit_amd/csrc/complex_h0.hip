@@ -20,7 +20,8 @@
 // by itself under the profiler: levels 1 and 2 19.0 with the matrix pipe 31% busy, level 3 12.8
 // with 20%), against 121 us with one thread per output point (k_cxh_level_lds: 40 us
 // per level, bound by a load of H0CX per multiply-add), which stays for a level of one
-// column per block (one-level operators, and level 1 under a dense sNDVR layer).
+// column per block (one-level operators, and level 1 under a dense sNDVR layer) and for
+// levels of a few points in many planes.
 #include "device_common.hpp"
 #include "solver_state.hpp"
 
@@ -406,6 +407,26 @@ static bool cx_tiles_fit(long nin, long n, long nz)
     return (nin + 1024) * (n + 1024) * 8 < 0x7fffffffL && (n + 1024) * (n + 1024) * 16 < 0x7fffffffL && nz <= 65535;
 }
 
+// Where the tiles pay, as in the real generic path: about 6 ns per workgroup and
+// chunk of 64 summed indices of the first pass, 2.5 ns per wave of a further level, against
+// 1 ps per multiply-add of k_cxh_level_lds and the launches that the first pass saves.
+// us of MYHX_CX with the first pass by tiles / by outputs: (4,4,12,12,12) with 16 vectors
+// 394 / 48, (1,50,20,20) with 16 547 / 66, (2,100,12,12,12) with 4 1,273 / 185, (32,32,10,10) with
+// 4 35 / 50; a further level of 2 points on 144 inner
+// ones 162 / 118, of 96 points 100 / 150.
+static bool cx_levels12_pays(long n1, long n2, long nz)
+{
+    const long ti = (n1 + 15) / 16, tc = (n2 + 15) / 16, tiles = ti * tc * nz, simds = 4L * g_num_cu;
+    const long k = 4 * tiles <= simds ? 4 : (2 * tiles <= simds ? 2 : 1);
+    const long wg = (ti * k + 3) / 4 * tc * nz, chunks = (n1 + 63) / 64 + (n2 + 63) / 64;
+    return wg * chunks * 6000 <= 8000000L + n1 * n2 * nz * (n1 + n2);
+}
+static bool cx_outer_pays(long P, long n, long nz)
+{
+    const long waves = ((P + 15) / 16) * ((n + 15) / 16) * nz;
+    return waves <= 4L * g_num_cu || waves * 2500 <= P * n * nz * n;
+}
+
 // waves per tile: as many as leave about one wave per SIMD
 static void launch_cxh_levels12(int n1, int n2, int nplane, int nvec, const dcx *h1, const dcx *h2, const dcx *dep2,
                                 long N, const double *res, double sh, const double *a, double sign, const double *x,
@@ -484,7 +505,8 @@ int hx_apply_cxh(scalit_ctx *c, int ntype, int nvec, const double *x, double *y,
     // the diagonal and levels 1 and 2 in one pass where both are level matrices
     int l = 0;
     if (c->sF >= 2 + (c->ndvr ? 1 : 0) && cx_tiles_fit(L[0].n, L[0].n, 1) &&
-        cx_tiles_fit(L[0].n, L[1].n, (long)L[1].blk * nvec)) {
+        cx_tiles_fit(L[0].n, L[1].n, (long)L[1].blk * nvec) &&
+        cx_levels12_pays(L[0].n, L[1].n, (long)L[1].blk * nvec)) {
         launch_cxh_levels12(L[0].n, L[1].n, L[1].blk, nvec, hcx(0), hcx(1), dcxp(1), N, c->res.p, sh, a, sign, x, y, s);
         l = 2;
     } else {
@@ -495,7 +517,7 @@ int hx_apply_cxh(scalit_ctx *c, int ntype, int nvec, const double *x, double *y,
         if (c->ndvr && l == c->sF - 1)
             hipLaunchKernelGGL(k_cxh_outh, dim3(cxh_grid((long)nin * n), nvec), dim3(256), 0, s, nin, n,
                                (const dcx *)c->outhcx.p, N, x, y);
-        else if (nin > 1 && cx_tiles_fit(nin, n, (long)blk * nvec))
+        else if (nin > 1 && cx_tiles_fit(nin, n, (long)blk * nvec) && cx_outer_pays(nin, n, (long)blk * nvec))
             hipLaunchKernelGGL(k_cxh_outer,
                                dim3((unsigned)((nin + 63) / 64), (unsigned)((n + 15) / 16), (unsigned)(blk * nvec)),
                                dim3(256), 0, s, nin, n, nvec, hcx(l), dcxp(l), N, x, y);

@@ -5,8 +5,9 @@
 //
 // Two paths:
 //  * generic: any number of levels and DEP pattern; the diagonal and levels 1
-//    and 2 in one MFMA pass, then one that adds to Y per further level (sizes
-//    past their 32-bit offsets, and one-level operators: thread per output).
+//    and 2 in one MFMA pass, then one that adds to Y per further level (levels
+//    of a few points in many planes, sizes past their 32-bit offsets, and one-level
+//    operators: thread per output).
 //  * fused 3-level path for sF=3, sDEP=(F,F,T) -- r, R, theta with
 //    DEP(r,R) x L^2_theta -- on FP64 / FP32 MFMA:
 //      pass A, one workgroup per (theta point, vector) slab S(n1 x n2) staged
@@ -366,6 +367,35 @@ static bool levels12_fits(long n1, long n2, long nplane, long nvec, size_t item)
     return (std::max(n1, n2) + 1024) * (std::max(n1, n2) + 1024) * (long)item < 0x7fffffffL && nplane * nvec <= 65535;
 }
 
+// Where the tile forms pay in the generic path.  Levels of a few points leave most
+// of a 16 x 16 tile empty, and thousands of planes make thousands of workgroups that each
+// cost the same: there the diagonal and the level go one thread per output.  The first
+// pass costs about 5 ns (FP32 2.5) per workgroup and chunk of 64 summed indices, the
+// form by outputs about 1 ps (0.6) per multiply-add and the launches that the one
+// pass saves (FP64 7 us); a further level 1 ns per wave against 0.5 ps per multiply-add,
+// so that a wave needs 2,000 of use (FP32 4,000; a full tile has 256 n), and up to a wave
+// per SIMD the two take the same.  us of the whole operator with the first pass by tiles / by outputs, FP64: (4,4,12,12,12) with 16 vectors 268
+// / 35, (2,2,20,20) with 16 67 / 18, (8,8,12,12,12) with 16 286 / 101, (17,17,20,20) with one
+// 15 / 19, (32,32,10,10) with 4 20 / 37, (2,2,10) with one 10 / 15; with a further level of
+// 2 points on 144 inner ones 142 / 107, of 96 points 79 / 194.  The rule's choice is within
+// 1.2 of the faster form in all but a few of the 1,484 and 3,254 shapes timed.
+template <typename T>
+static bool levels12_pays(long n1, long n2, long nz)
+{
+    const long ti = (n1 + 15) / 16, tc = (n2 + 15) / 16, tiles = ti * tc * nz, simds = 4L * g_num_cu;
+    // the workgroups of launch_levels12
+    const long wg = 4 * tiles <= simds ? tiles : nz * ((ti + 1) / 2) * (2 * tiles <= simds ? tc : (tc + 1) / 2);
+    const long chunks = (n1 + 63) / 64 + (n2 + 63) / 64;
+    return wg * chunks * (sizeof(T) == 8 ? 4750 : 4000) <=
+           (sizeof(T) == 8 ? 7000000L : 20000000L) + n1 * n2 * nz * (n1 + n2);
+}
+template <typename T>
+static bool outer_tiles_pay(long P, long n, long nz)
+{
+    const long waves = outer_tiles(P, n, nz);
+    return waves <= 4L * g_num_cu || waves * (sizeof(T) == 8 ? 2000 : 4000) <= P * n * nz * n;
+}
+
 template <typename T, typename S>
 static int hx_generic(scalit_ctx *c, const T *res, const T *shifts, T shift0, int nvec, const S *x, long ldx, S *y,
                       long ldy, bool transpose, const int *active, hipStream_t s)
@@ -386,7 +416,8 @@ static int hx_generic(scalit_ctx *c, const T *res, const T *shifts, T shift0, in
     // the diagonal and levels 1 and 2 in one pass where both are level matrices
     int l = 0;
     const Level *L = c->lv;
-    if (c->sF >= 2 + (c->ndvr ? 1 : 0) && levels12_fits(L[0].n, L[1].n, L[1].blk, nvec, sizeof(T))) {
+    if (c->sF >= 2 + (c->ndvr ? 1 : 0) && levels12_fits(L[0].n, L[1].n, L[1].blk, nvec, sizeof(T)) &&
+        levels12_pays<T>(L[0].n, L[1].n, (long)L[1].blk * nvec)) {
         launch_levels12<T, S, false>(L[0].n, L[1].n, L[1].blk, nvec, h[0], h[1], dep[1], res, shifts, shift0, x, ldx,
                                      y, ldy, active, s);
         l = 2;
@@ -396,7 +427,8 @@ static int hx_generic(scalit_ctx *c, const T *res, const T *shifts, T shift0, in
     for (; l < c->sF; l++) {
         if (c->ndvr && l == c->sF - 1)
             launch_h3x<T, S>(L[l].dim, L[l].n, nvec, outh_of<T>(c), transpose, x, ldx, y, ldy, active, s);
-        else if (l > 0 && outer_tiles_fit(L[l].dim, L[l].n, (long)L[l].blk * nvec, sizeof(T)))
+        else if (l > 0 && outer_tiles_fit(L[l].dim, L[l].n, (long)L[l].blk * nvec, sizeof(T)) &&
+                 outer_tiles_pay<T>(L[l].dim, L[l].n, (long)L[l].blk * nvec))
             launch_outer_tiles<T, S, S, true>(L[l].dim, L[l].n, nvec, h[l], 0, dep[l], x, ldx, y, ldy, active, s,
                                               L[l].blk);
         else

@@ -28,6 +28,8 @@ pytestmark = pytest.mark.gpu
     ((20, 24, 48), (1, 2), 4),     # 768 tiles: one wave
     ((6, 5, 4, 7), (1, 3), 3),
     ((3, 2, 130), (2,), 1),
+    ((4, 3, 30, 30), (1, 3), 5),   # small levels in many planes: one thread per output
+    ((8, 40, 2, 25), (2,), 2),     # and only the level of two points
 ])
 def test_complex_levels(sN, deps, nvec):
     g = P.rng(8)

@@ -33,6 +33,8 @@ SHAPES = [
     ((6, 5, 4, 7), (1, 3), 3),
     ((4, 3, 17, 5), (2, 3), 2),
     ((3, 2, 200), (2,), 3),
+    ((4, 3, 30, 30), (1, 3), 5),   # small levels in many planes: one thread per output
+    ((8, 40, 2, 25), (2,), 4),     # and only the level of two points
 ]
 
 
